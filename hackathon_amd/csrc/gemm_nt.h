@@ -31,3 +31,14 @@ int ql_gemm_nt2(int in_dtype, int c_dtype, int64_t M, int64_t N, int64_t K, cons
                 const void* B2, int64_t ldb2, int64_t K2, void* C, int64_t ldc, const void* bias,
                 float alpha, float beta, int splits, float* ws, hipStream_t s,
                 const void* residual = nullptr, int64_t ld_residual = 0);
+
+// The 4-bit linear for at most kSkinnyMaxRows rows of A (gemm_nf4_skinny.hip): qlora_gemm_nf4's
+// arguments, checked by it (K % 64 == 0, blocksize a power of two >= 64 dividing K, K2 0 or 64,
+// A 16-B aligned rows; log2 of the block sizes). No workspace.
+constexpr int64_t kSkinnyMaxRows = 32;
+int ql_gemm_nf4_skinny(int64_t M, int64_t N, int64_t K, const void* A, int64_t lda,
+                       const uint8_t* packed, const void* absmax, int nested, const float* code2,
+                       const float* absmax2, float offset, int log2_bs, int log2_bs2,
+                       const float* nf4_table, int64_t K2, const void* A2, int64_t lda2,
+                       const void* B2, int64_t ldb2, int in_dtype, void* C, int64_t ldc,
+                       const void* bias, float alpha, hipStream_t s);

@@ -1143,7 +1143,7 @@ int log2_exact(int64_t v) {  // log2 of a power of two, else -1
 }  // namespace
 
 extern "C" int64_t qlora_gemm_nf4_workspace_size(int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 0;
+  if (M <= kSkinnyMaxRows || N <= 0 || K <= 0 || K % BK) return 0;  // few rows: no split
   return ql_gemm_nt_workspace_floats(M, N, ql_gemm_nf4_auto_splits(M, N, K)) *
          (int64_t)sizeof(float);
 }
@@ -1172,6 +1172,10 @@ extern "C" int qlora_gemm_nf4(int64_t M, int64_t N, int64_t K, const void* A, in
     return QL_EALIGN;
   if (K2 > 0 && !ql_gemm_nt_fits(M, N, K2, A2, lda2, B2, ldb2)) return QL_EALIGN;
   if ((M + BM - 1) / BM * ((N + 255) / 256) >= (int64_t(1) << 30)) return QL_ESHAPE;
+  if (M <= kSkinnyMaxRows)
+    return ql_gemm_nf4_skinny(M, N, K, A, lda, packed, absmax, nested, code2, absmax2, offset,
+                              log2_bs, log2_bs2, nf4_table, K2, A2, lda2, B2, ldb2, in_dtype, C,
+                              ldc, bias, alpha, static_cast<hipStream_t>(stream));
   int splits = ql_gemm_nf4_auto_splits(M, N, K);
   const int64_t need = ql_gemm_nt_workspace_floats(M, N, splits) * (int64_t)sizeof(float);
   if (need > workspace_bytes || !workspace || !ql_aligned(workspace, 16)) splits = 1;
