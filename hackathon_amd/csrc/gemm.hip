@@ -303,7 +303,7 @@ int gemm_checked(int a_km, int b_kn, int64_t M, int64_t N, int64_t K, const void
     return QL_EALIGN;
   if (lda < (a_km ? M : K) || ldb < (b_kn ? N : K) || ldc < N) return QL_ESHAPE;
   if (!a_km && !b_kn && ql_gemm_nt_fits(M, N, K, A, lda, B, ldb)) {
-    int splits = ql_gemm_nt_auto_splits(M, N, K);
+    int splits = ql_gemm_nt_auto_splits(M, N, K, beta != 0.f);
     const int64_t need = ql_gemm_nt_workspace_floats(M, N, splits) * (int64_t)sizeof(float);
     if (need > ws_bytes || !ws || !ql_aligned(ws, 16)) splits = 1;
     return ql_gemm_nt(in_dtype, c_dtype, M, N, K, A, lda, B, ldb, C, ldc, bias, alpha, beta,
@@ -334,8 +334,9 @@ extern "C" int qlora_gemm(int a_km, int b_kn, int64_t M, int64_t N, int64_t K, c
 extern "C" int64_t qlora_gemm_workspace_size(int a_km, int b_kn, int64_t M, int64_t N,
                                              int64_t K) {
   if (a_km || b_kn || M <= 0 || N <= 0 || K <= 0 || K % 64) return 0;
-  return ql_gemm_nt_workspace_floats(M, N, ql_gemm_nt_auto_splits(M, N, K)) *
-         (int64_t)sizeof(float);
+  // enough for either beta: accumulating calls run the 256-row tile and its split count
+  const int plain = ql_gemm_nt_auto_splits(M, N, K), acc = ql_gemm_nt_auto_splits(M, N, K, true);
+  return ql_gemm_nt_workspace_floats(M, N, plain > acc ? plain : acc) * (int64_t)sizeof(float);
 }
 
 extern "C" int qlora_gemm_ws(int a_km, int b_kn, int64_t M, int64_t N, int64_t K, const void* A,

@@ -943,6 +943,29 @@ __global__ __launch_bounds__(256) void splitk_reduce(const float* __restrict__ w
   }
 }
 
+// The split-K sum: ws holds `nsplit` fp32 partials [M][N].
+template <int IT, int OT>
+int reduce_partials(const float* ws, int nsplit, void* C, int64_t ldc, const void* bias, int64_t M,
+                    int64_t N, float alpha, float beta, Residual res, hipStream_t s) {
+  using T = typename Elem<OT>::T;
+  const int64_t total = M * N;
+  if constexpr (OT != QL_F32) {
+    if (N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C & 7) == 0) {
+      int64_t grid = (total / 4 + 255) / 256;
+      if (grid > 256 * 16) grid = 256 * 16;
+      hipLaunchKernelGGL((splitk_reduce4<IT, OT>), dim3((unsigned)grid), dim3(256), 0, s, ws,
+                         nsplit, (uint16_t*)C, ldc, (const uint16_t*)bias, M, N, alpha, beta,
+                         res);
+      return ql_launch_status();
+    }
+  }
+  int64_t grid = (total + 255) / 256;
+  if (grid > 256 * 16) grid = 256 * 16;
+  hipLaunchKernelGGL((splitk_reduce<IT, OT>), dim3((unsigned)grid), dim3(256), 0, s, ws, nsplit,
+                     (T*)C, ldc, (const uint16_t*)bias, M, N, alpha, beta, res);
+  return ql_launch_status();
+}
+
 template <int IT, int OT, int NB, int BQ = kBDense>
 int launch(const void* A, int64_t lda, const void* B, int64_t ldb, const void* A2, int64_t lda2,
            const void* B2, int64_t ldb2, int64_t K2, void* C, int64_t ldc, const void* bias,
@@ -986,24 +1009,9 @@ int launch(const void* A, int64_t lda, const void* B, int64_t ldb, const void* A
                        (const uint16_t*)B2, ldb2, K2, (float*)nullptr, (int64_t)0, ws,
                        (const uint16_t*)nullptr, M, N, K, kps, 1.0f, 0.0f, false, nf4op,
                        Residual{});
-  int st = ql_launch_status();
+  const int st = ql_launch_status();
   if (st != QL_OK) return st;
-  const int64_t total = M * N;
-  if constexpr (OT != QL_F32) {
-    if (N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C & 7) == 0) {
-      int64_t grid = (total / 4 + 255) / 256;
-      if (grid > 256 * 16) grid = 256 * 16;
-      hipLaunchKernelGGL((splitk_reduce4<IT, OT>), dim3((unsigned)grid), dim3(256), 0, s, ws,
-                         nsplit, (uint16_t*)C, ldc, (const uint16_t*)bias, M, N, alpha, beta,
-                         res);
-      return ql_launch_status();
-    }
-  }
-  int64_t grid = (total + 255) / 256;
-  if (grid > 256 * 16) grid = 256 * 16;
-  hipLaunchKernelGGL((splitk_reduce<IT, OT>), dim3((unsigned)grid), dim3(256), 0, s, ws, nsplit,
-                     (T*)C, ldc, (const uint16_t*)bias, M, N, alpha, beta, res);
-  return ql_launch_status();
+  return reduce_partials<IT, OT>(ws, nsplit, C, ldc, bias, M, N, alpha, beta, res, s);
 }
 
 // Tile width for an M x N output: 224 when N is a multiple of 224, the output is large enough
@@ -1069,12 +1077,95 @@ int auto_splits_bn(int64_t M, int64_t N, int64_t K, int64_t bn) {
 
 }  // namespace
 
-int ql_gemm_nt_auto_splits(int64_t M, int64_t N, int64_t K) {
-  return auto_splits_bn(M, N, K, 32 * choose_nb(M, N));
+namespace {
+
+// Which kernel and how many splits of K. Times are modelled in microseconds from sweeps of every
+// tile over splits 1 .. 8 (M 64 .. 8192, N 512 .. 18944, K 896 .. 18944; weights rotated):
+//
+//   3 + rounds * (steps * step + tile) + (splits > 1: 3 + partials written and read at 6 TB/s)
+//
+//   tile       per CU  step   tile  fitted to (measured -> model)
+//   256 x 256     1    1.58    6    4096 x 18944 x 3584  479 -> 476 us
+//   256 x 224     1    1.43    6    4096 x 3584 x 3584    91 -> 90
+//   128 x 256     1    0.94    4    333 x 18944 x 3584    60 -> 60  (256 x 256: 96)
+//   128 x 128     1    0.456   4    1001 x 3584 x 3584    33 -> 33  (256 x 256, split: 56)
+//   64 x 128      2    0.59   2.5   4096 x 512 x 3584     24 -> 24  (256 x 256, split: 47)
+//
+// with the corrections the sweeps showed: a split 256 x 256 tile stores its partials row piece by
+// row piece, 12 us more (512 x 3584 x 18944 in 9: 96 us); several rounds of 128 x 128 run at 0.54
+// a step (8192 x 1536 x 4096: 120 us); one 64 x 128 workgroup per CU at 0.36; and the two small
+// tiles, which keep fewer loads in flight, lose a quarter where the operands are past what the
+// 256 MB cache holds beside its other work (64 x 128 at 512 x 18944 x 3584: 118 us). A smaller
+// tile is taken only where the model gives it 5%.
+struct Plan {
+  QlGemmTile tile;
+  int splits;
+};
+
+double reduce_us(int64_t M, int64_t N, int s) {
+  return s > 1 ? 3.0 + (s + 0.5) * double(M) * double(N) * 4.0 / 6.0e6 : 0.0;
 }
 
+double big_us(int64_t M, int64_t N, int64_t K, int s) {
+  const int nb = choose_nb(M, N);
+  const int64_t wgs = (M + BM - 1) / BM * ((N + 32 * nb - 1) / (32 * nb)) * s;
+  const double steps = double((K / BK + s - 1) / s);
+  return 3.0 + double((wgs + kCUs - 1) / kCUs) * (steps * (nb == 8 ? 1.58 : 1.43) + 6.0) +
+         (s > 1 ? 12.0 : 0.0) + reduce_us(M, N, s);
+}
+
+double mid_us(QlGemmTile tile, int64_t M, int64_t N, int64_t K, int s) {
+  const int64_t bm = tile == QlGemmTile::k64x128 ? 64 : 128;
+  const int64_t bn = tile == QlGemmTile::k128x256 ? 256 : 128;
+  const int64_t wgs = (M + bm - 1) / bm * ((N + bn - 1) / bn) * s;
+  const int64_t rounds = (wgs + kCUs - 1) / kCUs;
+  const double steps = double((K / BK + s - 1) / s);
+  const double cold = double(M + N) * double(K) * 2.0 > 100e6 ? 1.25 : 1.0;
+  double us;
+  if (tile == QlGemmTile::k128x256) {
+    us = 3.0 + double(rounds) * (steps * 0.94 + 4.0);
+  } else if (tile == QlGemmTile::k128x128) {
+    us = 3.0 + double(rounds) * (steps * cold * (rounds > 1 ? 0.54 : 0.456) + 4.0);
+  } else if (rounds <= 1) {
+    us = 4.0 + steps * cold * 0.36;
+  } else {  // two per CU: later workgroups start as earlier ones end
+    const double r = double(wgs) / double(2 * kCUs);
+    us = 3.0 + (r > 1.0 ? r : 1.0) * (steps * cold * 0.59 + 2.5);
+  }
+  return us + reduce_us(M, N, s);
+}
+
+// Up to this many rows the split count is the 256-row tile's, whatever tile runs: there the
+// forward multiplies by the packed NF4 weight (qlora_gemm_nf4, 256 x 256 tiles), and the same
+// product of the dequantised weight has to be the same sum.
+constexpr int64_t kNf4Rows = 256;
+
+Plan plan_nt(int64_t M, int64_t N, int64_t K) {
+  Plan best{QlGemmTile::k256, auto_splits_bn(M, N, K, 32 * choose_nb(M, N))};
+  double us = 0.95 * big_us(M, N, K, best.splits);
+  const int fixed = best.splits;
+  for (const QlGemmTile tile : {QlGemmTile::k128x128, QlGemmTile::k64x128, QlGemmTile::k128x256})
+    for (int s = M <= kNf4Rows ? fixed : 1; s <= (M <= kNf4Rows ? fixed : 16); ++s) {
+      if (s > 1 && M > kNf4Rows && K / BK / s < 6) break;
+      const double t = mid_us(tile, M, N, K, s);
+      if (t < us) {
+        us = t;
+        best = {tile, s};
+      }
+    }
+  return best;
+}
+
+}  // namespace
+
+int ql_gemm_nt_auto_splits(int64_t M, int64_t N, int64_t K, bool accumulate) {
+  return accumulate ? auto_splits_bn(M, N, K, 32 * choose_nb(M, N)) : plan_nt(M, N, K).splits;
+}
+
+// The same count as the dense product of these sizes, so that both are the same sum (beyond
+// kNf4Rows rows only callers that ask for it take the packed operand).
 int ql_gemm_nf4_auto_splits(int64_t M, int64_t N, int64_t K) {
-  return auto_splits_bn(M, N, K, 256);
+  return M <= kNf4Rows ? auto_splits_bn(M, N, K, 256) : plan_nt(M, N, K).splits;
 }
 
 int ql_gemm_nt2(int in_dtype, int c_dtype, int64_t M, int64_t N, int64_t K, const void* A,
@@ -1099,6 +1190,27 @@ int ql_gemm_nt2(int in_dtype, int c_dtype, int64_t M, int64_t N, int64_t K, cons
     u = K; K = K2; K2 = u;
   }
   if (K2 == 0) A2 = B2 = nullptr;
+  const Plan plan = plan_nt(M, N, K);
+  const int64_t ld_most = lda > ldb ? lda : ldb, ld2_most = K2 == 0 ? 0 : lda2 > ldb2 ? lda2 : ldb2;
+  if (plan.tile != QlGemmTile::k256 && plan.splits == splits && beta == 0.f &&
+      ld_most < kMidMaxLd && ld2_most < kMidMaxLd) {
+    const int64_t kps = ((K / BK + splits - 1) / splits) * BK;
+    const int nsplit = (int)((K + kps - 1) / kps);
+    const int st = ql_gemm_mid(plan.tile, in_dtype, c_dtype, M, N, K, A, lda, B, ldb, A2, lda2, B2,
+                               ldb2, K2, C, ldc, bias, alpha, kps, nsplit, ws, s, residual,
+                               ld_residual);
+    if (st != QL_OK || nsplit <= 1) return st;
+#define QL_GEMM_NT_REDUCE(ITC)                                                                \
+  QL_DISPATCH_DTYPE(c_dtype, OT,                                                              \
+                    return (reduce_partials<ITC, OT>(ws, nsplit, C, ldc, bias, M, N, alpha,   \
+                                                     beta, res, s)))
+    if (in_dtype == QL_BF16) {
+      QL_GEMM_NT_REDUCE(QL_BF16);
+    } else {
+      QL_GEMM_NT_REDUCE(QL_F16);
+    }
+#undef QL_GEMM_NT_REDUCE
+  }
   const bool narrow = choose_nb(M, N) == 7;
 #define QL_GEMM_NT_LAUNCH(ITC, NBC)                                                            \
   QL_DISPATCH_DTYPE(c_dtype, OT,                                                               \
