@@ -224,7 +224,9 @@ def tag(dtype: torch.dtype) -> int:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The handle of the current stream of t's device (torch.cuda.current_stream builds a Stream
+    object around it, 1.9 us against 0.1 a launch)."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
@@ -252,8 +254,16 @@ def require_rows(dtype: torch.dtype, **tensors: torch.Tensor | None) -> None:
             raise ValueError(f"{name} must be a 2-D matrix with unit stride along its rows")
 
 
+_I64X3 = ctypes.c_int64 * 3
+
+
 def i64_array(values) -> ctypes.Array:
     return (ctypes.c_int64 * len(values))(*[int(v) for v in values])
+
+
+def strides3(t: torch.Tensor) -> ctypes.Array:
+    """The first three strides of t."""
+    return _I64X3(*t.stride()[:3])
 
 
 class LoraFactor(ctypes.Structure):

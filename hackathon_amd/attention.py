@@ -20,8 +20,7 @@ from . import _common, _lib
 HEAD_DIM = 128
 
 
-def _strides3(t):
-    return _lib.i64_array([t.stride(0), t.stride(1), t.stride(2)])
+_strides3 = _lib.strides3
 
 
 def attn_fwd(q, k, v, scale, with_lse=True):

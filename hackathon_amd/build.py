@@ -3,7 +3,9 @@
 Every `csrc/*.hip` file is compiled by hipcc for gfx950 only (no other targets, no host
 fallback) and the objects are linked into `hackathon_amd/libqlora_gfx950.so`, which the
 Python façades load through ctypes. Run `python -m hackathon_amd.build` (or call
-`build()`); it always recompiles.
+`build()`); it always recompiles. The native host code of the fused layers
+(`csrc/host/host.cpp`, a CPython extension on torch's C++ API) is compiled by g++ into
+`hackathon_amd/_qlora_host.so` in the same call.
 
 Device flags:
   -O3 --offload-arch=gfx950
@@ -62,6 +64,32 @@ def _compile(src: Path) -> tuple[Path, str]:
     return obj, warn
 
 
+HOST_SOURCE = CSRC / "host" / "host.cpp"
+HOST_PATH = PKG / "_qlora_host.so"
+CXX = os.environ.get("CXX", shutil.which("g++") or "g++")
+
+
+def _build_host() -> Path:
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    torch_lib = Path(torch.__file__).resolve().parent / "lib"
+    includes = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    cmd = [CXX, "-O2", "-std=c++17", "-fPIC", "-shared",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f for i in includes for f in ("-isystem", str(i))], str(HOST_SOURCE), "-o", str(tmp),
+           "-L", str(torch_lib), "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10",
+           f"-Wl,-rpath,{torch_lib}"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"{CXX} failed for {HOST_SOURCE.name}:\n{' '.join(cmd)}\n{proc.stderr}")
+    os.replace(tmp, HOST_PATH)
+    return HOST_PATH
+
+
 def build(jobs: int | None = None, verbose: bool = False) -> Path:
     """Compile every csrc/*.hip for gfx950 and link the shared library. Returns its path."""
     BUILD.mkdir(exist_ok=True)
@@ -70,7 +98,9 @@ def build(jobs: int | None = None, verbose: bool = False) -> Path:
         raise RuntimeError(f"no HIP sources under {CSRC}")
     jobs = jobs or min(len(srcs), max(1, (os.cpu_count() or 2)))
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(_build_host)
         results = list(ex.map(_compile, srcs))
+        host.result()
     for obj, warn in results:
         if warn and verbose:
             print(f"[{obj.stem}] {warn}", file=sys.stderr)

@@ -47,7 +47,7 @@ import math
 
 import torch
 
-from . import _common, _lib, adapter_packs, attention, lora, nf4, rope, swiglu
+from . import _common, _host, _lib, adapter_packs, attention, lora, nf4, rope, swiglu
 from . import gemm as _gemm
 
 _PAD = 64  # padded LoRA K segment: up to 4 adapters of rank 16
@@ -119,72 +119,54 @@ def _t_buffer(rows, m, dtype, device):
     return torch.empty((rows, (m + 7) // 8 * 8), dtype=dtype, device=device)[:, :m]
 
 
-_NARROW = 2048  # projections narrower than this share a forward GEMM with their neighbours
-
-
-def _column_blocks(specs):
-    """[(first, last + 1)] projection ranges of the forward GEMMs over the shared output: a
-    wide projection gets its own GEMM (its column count then fills the 256-CU tile grid as it
-    does alone: 4096 x 3584 is exactly one wave of 256 x 224 tiles, where the 4096 x 4608 of
-    q|k|v would be 288 tiles of 256 x 256, two waves), narrow neighbours share one (k|v)."""
-    blocks, start, width = [], 0, 0
-    for i, s in enumerate(specs):
-        if i > start and (width + s.n > _NARROW or s.n > _NARROW or width > _NARROW):
-            blocks.append((start, i))
-            start, width = i, 0
-        width += s.n
-    blocks.append((start, len(specs)))
-    return blocks
+def _native_args(specs, ref):
+    """(weights, NF4 table, stream) of the native host calls for a group."""
+    return ([nf4.weight_args(s.packed, s.qs) for s in specs], nf4._nf4_table(ref.device),
+            _lib.stream_of(ref))
 
 
 def group_forward(x2, specs, ab, seeds=None):
     """y [M, sum n_g] = x2 W_cat^T + u sB_cat^T + bias, the state the backward needs and, with
-    dropout (specs' p > 0, one seed per adapter), (p, a16, [keep bits_g]), else None."""
+    dropout (specs' p > 0, one seed per adapter), (p, a16, [keep bits_g]), else None.
+    A projection wider than 2048 columns gets a GEMM of its own, narrow neighbours share one: the
+    7B q is exactly 256 tiles of 256 x 224 at 4096 rows, where q|k|v would be two waves."""
     dt = x2.dtype
     dev = x2.device
     M, K = x2.shape
     G = len(specs)
-    offs = _offsets(specs)
     a16, at, bs, bt = adapter_packs.pack_group(
         [(ab[2 * g], ab[2 * g + 1], specs[g].scaling) for g in range(G)], dt, _PAD)
+    p = specs[0].p
+    bias = _bias_cat(specs, dt, dev)
+    if M > nf4.FUSED_GEMM_MAX_ROWS or \
+            not all(nf4.fused_gemm_ok(s.qs, s.packed, x2) for s in specs):
+        weights, table, stream = _native_args(specs, x2)
+        y, ut, bitss = _host.load().group_forward(x2, a16, bs, weights, bias, p,
+                                                  _seed_words(seeds) if p > 0 else [], table,
+                                                  stream)
+        return y, (at, bt, ut), ((p, a16, bitss) if p > 0 else None)
+    # few rows: each projection's W dequantised inside its GEMM (bs rows of projection g
+    # are zero outside slot g, so u's other slots add nothing)
+    offs = _offsets(specs)
     u = torch.empty((M, _PAD), dtype=dt, device=dev)
     ut = _t_buffer(16 * G, M, dt, dev)
     drop = None
-    p = specs[0].p
-    if p > 0 and K % 64 == 0:
+    if p > 0:
         # each adapter's own mask of x (kept as bits) and its u, all adapters in one pass over x
         _, bitss = lora.dropout_down(x2, a16, p, seeds, u, ut)
-        drop = (p, a16, bitss)
-    elif p > 0:
-        # one adapter at a time: slot g's lora_down writes u columns 16 g .. 16 g + 15 and
-        # zeros after them, which the later slots overwrite
-        bitss = []
-        for g in range(G):
-            xd, bits = lora.dropout_with_bits(x2, p, seeds[g])
-            _gemm.lora_down(xd, a16[16 * g:16 * g + 16], u[:, 16 * g:],
-                            out_t=ut[16 * g:16 * g + 16])
-            bitss.append(bits)
         drop = (p, a16, bitss)
     else:
         _gemm.lora_down(x2, a16, u, out_t=ut)  # every slot in one pass over x
     y = torch.empty((M, offs[-1]), dtype=dt, device=dev)
-    bias = _bias_cat(specs, dt, dev)
-    if all(nf4.use_fused_gemm(x2, s.qs, s.packed, a2=u) for s in specs):
-        # few rows: each projection's W dequantised inside its GEMM (bs rows of projection g
-        # are zero outside slot g, so u's other slots add nothing)
-        for g, s in enumerate(specs):
-            c0, c1 = offs[g], offs[g + 1]
-            nf4.gemm_nf4(x2, s.packed, s.qs, out=y[:, c0:c1], a2=u, b2=bs[c0:c1],
-                         bias=None if bias is None else bias[c0:c1])
-        return y, (at, bt, ut), drop
-    w = torch.empty((offs[-1], K), dtype=dt, device=dev)
-    nf4.dequantize_nf4_group([(s.packed, s.qs) for s in specs], dt,
-                             [w[offs[g]:offs[g + 1]] for g in range(G)])
-    for p0, p1 in _column_blocks(specs):
-        c0, c1 = offs[p0], offs[p1]
-        _gemm.gemm_nt_cat(x2, w[c0:c1], u, bs[c0:c1], y[:, c0:c1],
-                          bias=None if bias is None else bias[c0:c1])
+    for g, s in enumerate(specs):
+        c0, c1 = offs[g], offs[g + 1]
+        nf4.gemm_nf4(x2, s.packed, s.qs, out=y[:, c0:c1], a2=u, b2=bs[c0:c1],
+                     bias=None if bias is None else bias[c0:c1])
     return y, (at, bt, ut), drop
+
+
+def _seed_words(seeds):
+    return [int(s) & 0xFFFF_FFFF_FFFF_FFFF for s in seeds]
 
 
 def group_backward(g, x2, at, bt, ut, specs, need_dx, need_ab, du_dut=None, db_given=None,
@@ -194,65 +176,12 @@ def group_backward(g, x2, at, bt, ut, specs, need_dx, need_ab, du_dut=None, db_g
     given, holds the adapters' down-projections of g already (du [M, 64], du^T [16 G, M]);
     `db_given`, the lora_B gradients [dB_0, dB_1, ..] already computed; `drop`, group_forward's
     dropout state."""
-    dt = g.dtype
-    dev = g.device
-    M = g.shape[0]
-    K = int(specs[0].qs.shape[1])
-    G = len(specs)
-    offs = _offsets(specs)
-    same_scaling = len({s.scaling for s in specs}) == 1
-    if du_dut is None:
-        du = torch.empty((M, _PAD), dtype=dt, device=dev)
-        dut = _t_buffer(16 * G, M, dt, dev)
-        if same_scaling:  # bt is block-diagonal: every adapter's du in one pass over g
-            _gemm.lora_down(g, bt, du, alpha=specs[0].scaling, out_t=dut)
-        else:
-            for i, s in enumerate(specs):
-                _gemm.lora_down(g[:, offs[i]:offs[i + 1]],
-                                bt[16 * i:16 * i + 16, offs[i]:offs[i + 1]], du[:, 16 * i:],
-                                alpha=s.scaling, out_t=dut[16 * i:16 * i + 16])
-    else:
-        du, dut = du_dut
-    dx = None
-    if need_dx:
-        wt = torch.empty((K, offs[-1]), dtype=dt, device=dev)
-        nf4.dequantize_nf4_t_group([(s.packed, s.qs) for s in specs], dt,
-                                   [wt[:, offs[i]:offs[i + 1]] for i in range(G)])
-        dx = torch.empty((M, K), dtype=dt, device=dev)
-        if drop is None:
-            _gemm.gemm_nt_cat(g, wt, du, at, dx)
-        else:
-            p, a16, bitss = drop
-            _gemm.gemm_nt_cat(g, wt, None, None, dx)
-            lora.up_masked_add_slots(dx, du, a16, bitss, p)  # every adapter in one pass
-        del wt
-    grads = []
-    da_all = None
-    if drop is not None and any(need_ab[0::2]):
-        # dA_g^T = du_g^T xd_g, each adapter on its own dropped input, all in one pass over x
-        # (xd_g formed from x and adapter g's keep bits)
-        da_all = _gemm.lora_wgrad_masked(dut, x2, drop[2], drop[0])
-        da_all = [da_all[16 * i:16 * i + 16] for i in range(G)]
-    elif drop is None and any(need_ab[0::2]):  # dA_g^T for every slot in one pass over x
-        da_all = _gemm.lora_wgrad(dut, x2, transposed=True)
-        da_all = [da_all[16 * i:16 * i + 16] for i in range(G)]
-    db_all = None
-    if db_given is None and sum(need_ab[1::2]) > 1:  # every dB_g in one pass over g
-        db_all = _gemm.lora_wgrad_diag(ut[:16 * G], g, offs, [s.scaling for s in specs])
-    for i, s in enumerate(specs):
-        da = db = None
-        if need_ab[2 * i]:
-            da = da_all[i]
-        if need_ab[2 * i + 1]:
-            if db_given is not None:
-                db = db_given[i]
-            elif db_all is not None:
-                db = db_all[offs[i]:offs[i + 1]]
-            else:
-                db = _gemm.lora_wgrad(ut[16 * i:16 * i + 16], g[:, offs[i]:offs[i + 1]],
-                                      alpha=s.scaling)
-        grads += [da, db]
-    return dx, grads
+    du, dut = du_dut or (None, None)
+    p, a16, bitss = drop or (0.0, None, [])
+    weights, table, stream = _native_args(specs, g)
+    return _host.load().group_backward(g, x2, at, bt, ut, weights, [s.scaling for s in specs],
+                                       bool(need_dx), list(need_ab), du, dut, db_given or [], p,
+                                       a16, list(bitss), table, stream)
 
 
 def _save(ctx, x2, drop, *tensors):
@@ -435,28 +364,24 @@ class LoraMLP(torch.autograd.Function):
                                               seeds[:2] if specs[0].p > 0 else None)
         n, N = specs[0].n, dspec.n
         a16_d, at_d, bs_d, bt_d = adapter_packs.pack(ab[4], ab[5], dspec.scaling, dt, _PAD)
-        h = torch.empty((M, n), dtype=dt, device=dev)
-        u_d = torch.empty((M, _PAD), dtype=dt, device=dev)
-        ut_d = _gemm.lora_t_buffer(M, dt, dev)
-        bits_d = swiglu.swiglu_fwd_lora_down(y[:, :n], y[:, n:], h, a16_d, u_d, ut_d,
-                                             p=dspec.p, seed=seeds[2] or 0)
-        out = torch.empty((M, N), dtype=dt, device=dev)
         bias = None if dspec.bias is None else dspec.bias.to(dt)
         res2 = None if residual is None else residual.view(M, N)
-        if nf4.use_fused_gemm(h, dspec.qs, dspec.packed, a2=u_d):  # W_d dequantised in-GEMM
+        if M > nf4.FUSED_GEMM_MAX_ROWS or not nf4.fused_gemm_ok(dspec.qs, dspec.packed):
+            (weight,), table, stream = _native_args((dspec,), y)
+            out, ut_d, bits_d = _host.load().mlp_down(
+                y, a16_d, bs_d, weight, bias, res2, dspec.p,
+                int(seeds[2] or 0) & 0xFFFF_FFFF_FFFF_FFFF, table, stream)
+        else:  # few rows: W_d dequantised in the GEMM
+            h = torch.empty((M, n), dtype=dt, device=dev)
+            u_d = torch.empty((M, _PAD), dtype=dt, device=dev)
+            ut_d = _gemm.lora_t_buffer(M, dt, dev)
+            bits_d = swiglu.swiglu_fwd_lora_down(y[:, :n], y[:, n:], h, a16_d, u_d, ut_d,
+                                                 p=dspec.p, seed=seeds[2] or 0)
+            out = torch.empty((M, N), dtype=dt, device=dev)
             nf4.gemm_nf4(h, dspec.packed, dspec.qs, out=out, a2=u_d, b2=bs_d, bias=bias)
             if res2 is not None:
                 out = res2 + out
-        else:
-            w = nf4.dequantize_nf4(dspec.packed, dspec.qs, dt)
-            if res2 is not None and bias is None:
-                _gemm.gemm_nt_cat(h, w, u_d, bs_d, out, residual=res2)
-            else:
-                _gemm.gemm_nt_cat(h, w, u_d, bs_d, out, bias=bias)
-                if res2 is not None:
-                    out = res2 + out
-            del w
-        del h, u_d
+            del h, u_d
         saved = [x2, y, at, bt, ut, at_d, bt_d, ut_d]
         ctx.drop_d = bits_d is not None
         if ctx.drop_d:
@@ -481,9 +406,9 @@ class LoraMLP(torch.autograd.Function):
             t = t[2:]
         drop = None if ctx.n_drop == 0 else (ctx.p, t[0], t[1:1 + ctx.n_drop])
         specs, dspec = ctx.specs, ctx.dspec
-        dt, dev = x2.dtype, x2.device
+        dt = x2.dtype
         M = x2.shape[0]
-        n, N = specs[0].n, dspec.n
+        N = dspec.n
         # x, specs, dspec, seeds, residual, A_gate, B_gate, A_up, B_up, A_d, B_d
         need = ctx.needs_input_grad
         dres = dout if need[4] else None
@@ -492,31 +417,12 @@ class LoraMLP(torch.autograd.Function):
             dy = dy.to(dt)
         if dy.stride(-1) != 1 or dy.stride(0) % 8 or dy.data_ptr() % 16:
             dy = dy.contiguous()
-        s_d = dspec.scaling
-        du_d = torch.empty((M, _PAD), dtype=dt, device=dev)
-        dut_d = _gemm.lora_t_buffer(M, dt, dev)
-        _gemm.lora_down(dy, bt_d, du_d, alpha=s_d, out_t=dut_d)  # du_d = s_d dY B_d
-        wt = nf4.dequantize_nf4_t(dspec.packed, dspec.qs, dt)    # W_d^T [n, N]
-        dh = torch.empty((M, n), dtype=dt, device=dev)
-        if bits_d is None:
-            _gemm.gemm_nt_cat(dy, wt, du_d, at_d, dh)
-        else:  # the adapter term goes through its mask of h inside the SwiGLU backward
-            _gemm.gemm_nt_cat(dy, wt, None, None, dh)
-        del wt
-        db_d = _gemm.lora_wgrad(ut_d, dy, alpha=s_d) if need[10] else None
-        g = torch.empty((M, 2 * n), dtype=dt, device=dev)
-        du = torch.empty((M, _PAD), dtype=dt, device=dev)
-        dut = _t_buffer(32, M, dt, dev)
-        gate_s, up_s = specs
-        db_g, db_u, da_d = swiglu.swiglu_bwd_lora(
-            dh, y[:, :n], y[:, n:], g[:, :n], g[:, n:], bt[:16, :n], bt[16:32, n:], ut[:16], ut[16:32],
-            gate_s.scaling, up_s.scaling, gate_s.scaling, up_s.scaling, du, dut, ud_t=dut_d,
-            bits_down=bits_d, p_down=dspec.p,
-            du_add=None if bits_d is None else du_d, a_add=None if bits_d is None else a16_d)
-        del dh, du_d
-        dx, grads = group_backward(g, x2, at, bt, ut, specs, need[0], need[5:9],
-                                   du_dut=(du, dut), db_given=[db_g, db_u], drop=drop)
-        grads = grads + [da_d if need[9] else None, db_d]
+        p, a16, bitss = drop or (0.0, None, [])
+        weights, table, stream = _native_args((*specs, dspec), dy)
+        dx, grads = _host.load().mlp_backward(
+            dy, x2, y, at, bt, ut, weights[:2], [s.scaling for s in specs], p, a16, list(bitss),
+            at_d, bt_d, ut_d, weights[2], dspec.scaling, dspec.p, a16_d, bits_d, need[0],
+            list(need[5:11]), table, stream)
         grads = [None if gr is None else gr.to(t_) for gr, t_ in zip(grads, ctx.ab_dtypes)]
         return (None if dx is None else dx.view(ctx.shape)), None, None, None, dres, *grads
 

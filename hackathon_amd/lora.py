@@ -24,7 +24,7 @@ import math
 
 import torch
 
-from . import _common, _lib, adapter_packs
+from . import _common, _host, _lib, adapter_packs
 from . import gemm as _gemm
 
 TORCH_DROPOUT_RNG = False
@@ -253,26 +253,24 @@ class LoraNF4Linear(torch.autograd.Function):
         N = int(quant_state.shape[0])
         # A, A^T|0, s*B|0 and B^T in the compute dtype, one launch (kept for the backward)
         a16, at, bs, bt = adapter_packs.pack(a_weight, b_weight, scaling, dt, _PAD)
-        u = torch.empty((M, _PAD), dtype=dt, device=x2.device)
-        ut = _gemm.lora_t_buffer(M, dt, x2.device)                     # u^T, for dB
-        bits = None
-        if p > 0 and K % 64 == 0:  # the keep bits and u in one pass over x
-            _, (bits,) = dropout_down(x2, a16, p, (seed,), u, ut)
-        elif p > 0:
-            xd, bits = dropout_with_bits(x2, p, seed)
-            _gemm.lora_down(xd, a16, u, out_t=ut)
-            del xd
-        else:
-            _gemm.lora_down(x2, a16, u, out_t=ut)
-        y = torch.empty((M, N), dtype=dt, device=x2.device)
         b16 = None if bias is None else bias.to(dt)
-        if nf4.use_fused_gemm(x2, quant_state, packed, a2=u):  # few rows: W dequantised in-GEMM
-            nf4.gemm_nf4(x2, packed, quant_state, out=y, a2=u, b2=bs, bias=b16)
-        else:
-            w = nf4.dequantize_nf4(packed, quant_state, dt)
-            _gemm.gemm_nt_cat(x2, w, u, bs, y, bias=b16)
-            del w
-        del u
+        bits = None
+        if M > nf4.FUSED_GEMM_MAX_ROWS or not nf4.fused_gemm_ok(quant_state, packed, x2):
+            y, ut, bitss = _host.load().group_forward(
+                x2, a16, bs, [nf4.weight_args(packed, quant_state)], b16, float(p),
+                [int(seed) & 0xFFFF_FFFF_FFFF_FFFF] if p > 0 else [],
+                nf4._nf4_table(x2.device), _lib.stream_of(x2))
+            if p > 0:
+                (bits,) = bitss
+        else:  # few rows: W dequantised in the GEMM
+            u = torch.empty((M, _PAD), dtype=dt, device=x2.device)
+            ut = _gemm.lora_t_buffer(M, dt, x2.device)                 # u^T, for dB
+            if p > 0:  # the keep bits and u in one pass over x
+                _, (bits,) = dropout_down(x2, a16, p, (seed,), u, ut)
+            else:
+                _gemm.lora_down(x2, a16, u, out_t=ut)
+            y = nf4.gemm_nf4(x2, packed, quant_state, a2=u, b2=bs, bias=b16)
+            del u
         ctx.save_for_backward(x2, ut, at, bt, a16 if p > 0 else None, bits)
         ctx.packed, ctx.quant_state, ctx.scaling = packed, quant_state, float(scaling)
         ctx.p = float(p)
@@ -290,30 +288,17 @@ class LoraNF4Linear(torch.autograd.Function):
         if g2.dtype != dt:
             g2 = g2.to(dt)
         g2 = g2.contiguous()
-        s = ctx.scaling
-        du = torch.empty((M, _PAD), dtype=dt, device=g2.device)
-        dut = _gemm.lora_t_buffer(M, dt, g2.device)
-        _gemm.lora_down(g2, bt, du, alpha=s, out_t=dut)                 # du = s g B
-        dx = da = db = None
-        if ctx.needs_input_grad[0]:
-            wt = nf4.dequantize_nf4_t(ctx.packed, ctx.quant_state, dt)  # [K, N]
-            dx = torch.empty((M, K), dtype=dt, device=g2.device)
-            if bits is None:
-                _gemm.gemm_nt_cat(g2, wt, du, at, dx)
-            else:
-                _gemm.gemm_nt_cat(g2, wt, None, None, dx)
-                up_masked_add(dx, du, a16, bits, ctx.p)
-            del wt
+        need = ctx.needs_input_grad
+        dx, (da, db) = _host.load().group_backward(
+            g2, x2, at, bt, ut, [nf4.weight_args(ctx.packed, ctx.quant_state)], [ctx.scaling],
+            need[0], [need[1], need[2]], None, None, [], ctx.p, a16,
+            [] if bits is None else [bits], nf4._nf4_table(g2.device), _lib.stream_of(g2))
+        if dx is not None:
             dx = dx.view(ctx.shape)
-        if ctx.needs_input_grad[1]:                                     # [16, K] = du^T xd
-            da = (_gemm.lora_wgrad(dut, x2, transposed=True) if bits is None
-                  else _gemm.lora_wgrad_masked(dut, x2, [bits], ctx.p))  # xd from x and bits
-            if da.dtype != ctx.wdtypes[0]:
-                da = da.to(ctx.wdtypes[0])
-        if ctx.needs_input_grad[2]:
-            db = _gemm.lora_wgrad(ut, g2, alpha=s)                     # [N, 16] = s g^T u
-            if db.dtype != ctx.wdtypes[1]:
-                db = db.to(ctx.wdtypes[1])
+        if da is not None and da.dtype != ctx.wdtypes[0]:
+            da = da.to(ctx.wdtypes[0])
+        if db is not None and db.dtype != ctx.wdtypes[1]:
+            db = db.to(ctx.wdtypes[1])
         return dx, da, db, None, None, None, None, None, None
 
 

@@ -80,6 +80,15 @@ def _scale_args(quant_state):
     return absmax, 0, None, None, 0.0, 1
 
 
+def weight_args(packed, quant_state):
+    """The weight as the native host code takes it: (packed, absmax, nested, code2, absmax2,
+    offset, blocksize, blocksize2, rows, cols)."""
+    absmax, nested, code2, absmax2, offset, blocksize2 = _scale_args(quant_state)
+    rows, cols = quant_state.shape
+    return (packed.contiguous(), absmax, nested, code2, absmax2, offset, int(quant_state.blocksize),
+            blocksize2, int(rows), int(cols))
+
+
 def dequantize_nf4(packed, quant_state, dtype=torch.float16, out=None):
     """The weight [out_features, in_features] in `dtype`, from the packed NF4 bytes
     (solution/nf4.py:71-92)."""

@@ -17,8 +17,7 @@ import torch
 from . import _common, _lib
 
 
-def _strides(t):
-    return _lib.i64_array((t.stride(0), t.stride(1), t.stride(2)))
+_strides = _lib.strides3
 
 
 def _launch(q, k, cos, sin, q_out, k_out, backward):
