@@ -1093,8 +1093,9 @@ namespace {
 //
 // with the corrections the sweeps showed: a split 256 x 256 tile stores its partials row piece by
 // row piece, 12 us more (512 x 3584 x 18944 in 9: 96 us); several rounds of 128 x 128 run at 0.54
-// a step (8192 x 1536 x 4096: 120 us); one 64 x 128 workgroup per CU at 0.36; and the two small
-// tiles, which keep fewer loads in flight, lose a quarter where the operands are past what the
+// a step (8192 x 1536 x 4096: 120 us), of 64 x 128 at 0.75 (2048 x 8960 x 1536 between a layer's
+// other kernels: 98 us against 86 for 256 x 224; alone 74 against 78); one 64 x 128 workgroup per
+// CU at 0.36; and the two small tiles, which keep fewer loads in flight, lose a quarter where the operands are past what the
 // 256 MB cache holds beside its other work (64 x 128 at 512 x 18944 x 3584: 118 us). A smaller
 // tile is taken only where the model gives it 5%.
 struct Plan {
@@ -1130,7 +1131,7 @@ double mid_us(QlGemmTile tile, int64_t M, int64_t N, int64_t K, int s) {
     us = 4.0 + steps * cold * 0.36;
   } else {  // two per CU: later workgroups start as earlier ones end
     const double r = double(wgs) / double(2 * kCUs);
-    us = 3.0 + (r > 1.0 ? r : 1.0) * (steps * cold * 0.59 + 2.5);
+    us = 3.0 + (r > 1.0 ? r : 1.0) * (steps * cold * (r > 1.0 ? 0.75 : 0.59) + 2.5);
   }
   return us + reduce_us(M, N, s);
 }
