@@ -108,6 +108,9 @@ _SIGNATURES = {
     "qlora_gemm_nf4": [_c_i64, _c_i64, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_ptr,
                        _c_ptr, _c_f32, _c_int, _c_int, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr,
                        _c_i64, _c_int, _c_ptr, _c_i64, _c_ptr, _c_f32, _c_ptr, _c_i64, _c_ptr],
+    "qlora_nf4_lora_few": [_c_i64, _c_i64, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_ptr,
+                           _c_ptr, _c_f32, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_f32, _c_int,
+                           _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_ptr],
     "qlora_lora_wgrad_diag": [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64, _c_int, _c_int,
                               _c_i64p, ctypes.POINTER(ctypes.c_float), _c_ptr, _c_ptr, _c_i64,
                               _c_ptr],
@@ -145,6 +148,7 @@ _SIZE_QUERIES = {
     "qlora_gemm_workspace_size": [_c_int, _c_int, _c_i64, _c_i64, _c_i64],
     "qlora_gemm_nt_cat_workspace_size": [_c_i64, _c_i64, _c_i64],
     "qlora_gemm_nf4_workspace_size": [_c_i64, _c_i64, _c_i64],
+    "qlora_nf4_lora_few_workspace_size": [_c_i64, _c_i64],
     "qlora_lora_down_workspace_size": [_c_i64, _c_i64, _c_int],
     "qlora_lora_dropout_down_workspace_size": [_c_i64, _c_i64, _c_int],
     "qlora_lora_wgrad_workspace_size": [_c_i64, _c_i64, _c_int],

@@ -302,6 +302,37 @@ class LoraNF4Linear(torch.autograd.Function):
         return dx, da, db, None, None, None, None, None, None
 
 
+class LoraNF4Few(torch.autograd.Function):
+    """LoraNF4Linear's forward where no gradient is wanted, for a few rows: two launches that read
+    the adapter's fp32 factors as they are (qlora_nf4_lora_few), instead of packing them, the
+    down-projection, its reduce and the GEMM. Decoding calls this per token."""
+
+    @staticmethod
+    def forward(ctx, x, a_weight, b_weight, packed, quant_state, bias, scaling):
+        from . import nf4
+
+        x2 = x.reshape(-1, x.shape[-1])
+        y = nf4.lora_few(x2, packed, quant_state, a_weight, b_weight, scaling,
+                         None if bias is None else bias.to(x.dtype))
+        return y.view(*x.shape[:-1], y.shape[-1])
+
+
+def _takes_few(x, a_w, b_w, packed, qs):
+    """Whether LoraNF4Few takes this call: at most 32 rows, no gradient wanted, contiguous fp32
+    factors, operands the kernel's 16-B loads can read."""
+    from . import nf4
+
+    K = x.shape[-1]
+    if not 0 < x.numel() <= nf4.LORA_FEW_MAX_ROWS * K or not x.is_contiguous():
+        return False
+    if torch.is_grad_enabled() and (x.requires_grad or a_w.requires_grad or b_w.requires_grad):
+        return False
+    return (a_w.dtype == torch.float32 and b_w.dtype == torch.float32 and a_w.is_contiguous()
+            and b_w.is_contiguous() and packed.is_contiguous() and a_w.data_ptr() % 16 == 0
+            and b_w.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0
+            and nf4.fused_gemm_ok(qs, packed))
+
+
 def _fused_base(layer, adapter, x, compute_dtype, p):
     """(packed, quant_state, bias) when the layer can run as LoraNF4Linear, else None: rank
     16, a frozen NF4 base whose shapes the k-contiguous kernels take, dropout off or drawn
@@ -366,6 +397,11 @@ def lora_forward(self, x, *args, **kwargs):
     if fused is not None:
         weight, qs, bias = fused
         xc = x if x.dtype == compute_dtype else x.to(compute_dtype)
+        a_w, b_w = self.lora_A[adapter].weight, self.lora_B[adapter].weight
+        if p == 0 and _takes_few(xc, a_w, b_w, weight, qs):
+            y = LoraNF4Few.apply(xc, a_w, b_w, weight, qs, bias, self.scaling[adapter])
+            out_dtype = torch.promote_types(x.dtype, compute_dtype)
+            return y if y.dtype == out_dtype else y.to(out_dtype)
         with torch.autocast("cuda", enabled=False):
             y = LoraNF4Linear.apply(xc, self.lora_A[adapter].weight, self.lora_B[adapter].weight,
                                     weight, qs, bias, self.scaling[adapter], p,

@@ -263,6 +263,25 @@ def gemm_nf4(x, packed, quant_state, out=None, a2=None, b2=None, bias=None, alph
     return out
 
 
+LORA_FEW_MAX_ROWS = 32  # qlora_nf4_lora_few's row limit
+
+
+def lora_few(x, packed, quant_state, lora_a, lora_b, scaling, bias=None):
+    """x @ W^T + bf16(x @ A^T) @ (scaling B)^T (+ bias) for x [M <= 32, K] and an adapter's fp32
+    factors A [16, K], B [N, 16], in two launches (qlora_nf4_lora_few)."""
+    M, K = x.shape
+    absmax, nested, code2, absmax2, offset, blocksize2 = _scale_args(quant_state)
+    N = int(quant_state.shape[0])
+    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    ws, ws_bytes = _lib.workspace("qlora_nf4_lora_few_workspace_size", M, K, device=x.device)
+    _lib.call("qlora_nf4_lora_few", M, N, K, x.data_ptr(), x.stride(0), packed.data_ptr(),
+              absmax.data_ptr(), nested, _lib.ptr(code2), _lib.ptr(absmax2), offset,
+              int(quant_state.blocksize), blocksize2, _nf4_table(packed.device).data_ptr(),
+              lora_a.data_ptr(), lora_b.data_ptr(), float(scaling), _lib.tag(x.dtype),
+              out.data_ptr(), N, _lib.ptr(bias), _lib.ptr(ws), ws_bytes, _lib.stream_of(x))
+    return out
+
+
 def transposed_dequant_ok(quant_state, packed=None):
     """Whether dequantize_nf4_t takes this weight: in_features % 128 == 0,
     out_features % 8 == 0, blocksize a power of two >= 16 (and, when given, the packed codes

@@ -479,9 +479,10 @@ int qlora_gemm_nt_cat_residual(int64_t M, int64_t N, int64_t K, const void* A, i
  *   C[M,N] = alpha * (A[M,K] W[N,K]^T + A2[M,K2] B2[N,K2]^T) (+ bias[n]),  C in in_dtype,
  * where W is the weight qlora_nf4_dequant produces from (packed, absmax, nested, code2,
  * absmax2, offset, blocksize, blocksize2, nf4_table) for n_weights = N * K, rounded to
- * in_dtype: the products see exactly those 16-bit values, so C equals qlora_gemm_nt_cat on
- * the dequantised W bit for bit. W's packed bytes are read once per 256-row tile of A instead
- * of writing and re-reading a dense 16-bit copy.
+ * in_dtype: the products see exactly those 16-bit values. Above 32 rows C equals
+ * qlora_gemm_nt_cat on the dequantised W bit for bit, and W's packed bytes are read once per
+ * 256-row tile of A instead of writing and re-reading a dense 16-bit copy; up to 32 rows a kernel
+ * without tiles sums the same products in another order of k.
  * K % 64 == 0; blocksize a power of two >= 64 dividing K (blocksize2 a power of two when
  * nested); K2 % 64 == 0 and K2 <= 128 (the rank-16 LoRA segment, zero-padded to 64 columns,
  * as in qlora_gemm_nt_cat); A, packed 16-B aligned, lda >= K a multiple of 8; A2/B2 as in
@@ -498,6 +499,24 @@ int qlora_gemm_nf4(int64_t M, int64_t N, int64_t K, const void* A, int64_t lda,
                    const void* B2, int64_t ldb2, int in_dtype, void* C, int64_t ldc,
                    const void* bias, float alpha, void* workspace, int64_t workspace_bytes,
                    ql_stream_t stream);
+
+/*
+ * A 4-bit LoRA linear (rank 16, no dropout) for at most 32 rows, in two launches:
+ *   C[M,N] = x[M,K] W[N,K]^T + u (scaling B)^T (+ bias[n]),  u = x A^T rounded to dtype,
+ * W as in qlora_gemm_nf4, the adapter's factors read as they are trained: lora_a [16, K] and
+ * lora_b [N, 16] in fp32 (contiguous, 16-B aligned), each value (scaling B after the product)
+ * rounded to dtype where it is used, as qlora_lora_pack rounds it. K, blocksizes, x, packed, C and
+ * bias as in qlora_gemm_nf4; M > 32 returns QL_ESHAPE. Workspace (16-B aligned,
+ * qlora_nf4_lora_few_workspace_size bytes, required): the partial sums of u.
+ * Replaces: solution/lora.py:157-173 over solution/nf4.py:95-102, without gradients.
+ */
+int64_t qlora_nf4_lora_few_workspace_size(int64_t M, int64_t K);
+int qlora_nf4_lora_few(int64_t M, int64_t N, int64_t K, const void* x, int64_t ldx,
+                       const uint8_t* packed, const void* absmax, int nested, const float* code2,
+                       const float* absmax2, float offset, int blocksize, int blocksize2,
+                       const float* nf4_table, const float* lora_a, const float* lora_b,
+                       float scaling, int dtype, void* C, int64_t ldc, const void* bias,
+                       void* workspace, int64_t workspace_bytes, ql_stream_t stream);
 
 /*
  * LoRA down-projection (rank 16) for `slots` = G adapters (1 <= G <= 4) that share X:

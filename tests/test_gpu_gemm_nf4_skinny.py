@@ -1,4 +1,4 @@
-"""qlora_gemm_nf4 for a few rows (the decode path, up to 32 rows): the 4-bit linear whose
+"""qlora_gemm_nf4 and qlora_nf4_lora_few for a few rows (the decode path, up to 32 rows): the 4-bit linear whose
 workgroups hold 16 or 32 weight rows and split K over their waves, against an fp64 product of
 the weight qlora_nf4_dequant writes, at the edges of its tiles."""
 
@@ -62,3 +62,61 @@ def test_few_rows_zero_weight_past_k_meets_no_inf():
     got = nf4.gemm_nf4(x, packed, st)
     assert torch.equal(got[1], nf4.gemm_nf4(x[1:], packed, st)[0])
     assert torch.equal(got[0].isnan(), (x[:1].double() @ w.double().t())[0].isnan())
+
+@pytest.mark.parametrize("M,N,K,nested,dtype,bias", [
+    (1, 64, 128, True, torch.bfloat16, False),
+    (4, 18944, 3584, True, torch.bfloat16, True),
+    (16, 576, 18944, True, torch.float16, True),     # eight splits of the down-projection
+    (17, 4864, 896, False, torch.bfloat16, False),   # second group of x rows
+    (32, 8256, 1536, True, torch.float16, True),
+])
+def test_lora_few_against_fp64(M, N, K, nested, dtype, bias):
+    """qlora_nf4_lora_few: the whole 4-bit LoRA linear from the fp32 factors, u and s B rounded to
+    the compute dtype where the layer rounds them."""
+    print(f"lora_few M={M} N={N} K={K} nested={nested} {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    packed, st = quant.quantize_nf4(torch.randn(N, K, device="cuda", generator=g) * 0.02, 64,
+                                    compress_statistics=nested)
+    x = torch.randn(M, K, device="cuda", generator=g).to(dtype)
+    a = torch.randn(16, K, device="cuda", generator=g) / K ** 0.5
+    b = torch.randn(N, 16, device="cuda", generator=g) * 0.05
+    bb = torch.randn(N, device="cuda", generator=g).to(dtype) if bias else None
+    got = nf4.lora_few(x, packed, st, a, b, 2.0, bb)
+    w = nf4.dequantize_nf4(packed, st, dtype).double()
+    ulp16 = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    a16, sb = a.to(dtype).double(), (2.0 * b).to(dtype).double()
+    u = x.double() @ a16.t()
+    ref = x.double() @ w.t() + u @ sb.t()
+    mag = x.double().abs() @ w.abs().t() + (x.double().abs() @ a16.abs().t()) @ sb.abs().t()
+    if bias:
+        ref += bb.double()
+    # fp32 accumulation over K + 16 terms, u rounded once, then one rounding to the output
+    bound = ((K + 32) * 2.0 ** -24 * mag + ulp16 * (u.abs() @ sb.abs().t()) + ulp16 * ref.abs()
+             + 1e-6)
+    assert torch.all((got.double() - ref).abs() <= bound)
+
+
+def test_layer_takes_the_few_row_kernel_only_without_gradients(monkeypatch):
+    from hackathon_amd import lora
+
+    base = quant.Linear4bit.from_weight(torch.randn(256, 128, device="cuda").bfloat16(),
+                                        compute_dtype=torch.bfloat16)
+    layer = lora.LoraLinear4bit(base, compute_dtype=torch.bfloat16, init_b_std=0.05)
+    calls = []
+    real = nf4.lora_few
+    monkeypatch.setattr(nf4, "lora_few", lambda *a, **k: (calls.append(1), real(*a, **k))[1])
+    x = torch.randn(3, 2, 128, device="cuda").bfloat16()
+    y = layer(x)
+    y.float().sum().backward()
+    assert not calls and layer.lora_B["default"].weight.grad is not None
+    with torch.no_grad():
+        z = layer(x)
+        assert len(calls) == 1 and z.shape == y.shape and not z.requires_grad
+        # another order of the same fp32 sums, one 16-bit rounding either way
+        assert torch.allclose(z.float(), y.float(), rtol=2.0 ** -7, atol=1e-2)
+        layer(torch.randn(33, 128, device="cuda").bfloat16())           # a row too many
+        layer(torch.randn(2, 256, device="cuda").bfloat16()[:, ::2])    # strided x
+        assert len(calls) == 1
+        layer.lora_A["default"].to(torch.bfloat16)                       # not fp32 factors
+        layer(x)
+        assert len(calls) == 1
