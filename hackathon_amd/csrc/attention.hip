@@ -157,49 +157,70 @@ QL_DEV uint4 frag_tr(const char* __restrict__ t, int r0, int c0, int fq, int fr)
 // elements; rows past S re-read row S - 1) by the 4 waves of a workgroup: load i of wave w
 // fills tile rows 4p .. 4p + 3 with p = 4 i + w; lane l writes LDS bytes [16 l, 16 l + 16) of
 // that 1 KiB span, i.e. row 4p + l / 16, physical chunk l % 16, which holds the logical chunk
-// the swizzle maps there (an XOR is its own inverse). Row 4p + l / 16 has row & 15 =
-// 4 w + l / 16 for every load, so the lane's byte offset from the span's first row is fixed:
-// each load is a wave-uniform base (SGPRs) plus that offset.
-// One direct-to-LDS load (16 B per lane from sbase + voff, lane l writing LDS bytes
-// [lds + 16 l, lds + 16 l + 16)), written as inline assembly: the compiler's wait-count pass
-// treats a pending direct-to-LDS load as an out-of-order LDS-counter event and then drains
-// every LDS read (lgkmcnt(0)) before each product that uses one; with the load hidden from
-// it, fragment reads are waited for in order, so reads issued ahead stay in flight. Nothing
-// waits for these loads but wait_all_barrier, which every kernel runs before it reads a tile
-// it loaded. (s_nop 4: the wait states a write of M0, or a VALU write of an address SGPR,
-// needs before a vector memory load reads it; inline assembly gets no hazard padding.)
+// the swizzle maps there (an XOR is its own inverse; row 4p + l / 16 has row & 15 =
+// 4 w + l / 16 for every load).
+// The loads are written as inline assembly: the compiler's wait-count pass treats a pending
+// direct-to-LDS load as an out-of-order LDS-counter event and then drains every LDS read
+// (lgkmcnt(0)) before each product that uses one; with the load hidden from it, fragment reads
+// are waited for in order, so reads issued ahead stay in flight. Nothing waits for these loads
+// but wait_all_barrier, which every kernel runs before it reads a tile it loaded. (s_nop 4: the
+// wait states a VALU write of an address SGPR, or a write of M0, needs before a vector memory
+// load reads it; s_nop 0: those of a scalar write of M0. Inline assembly gets no hazard
+// padding.)
+// A tile inside the tensor is one block of assembly: one scalar base, four lane offsets kept in
+// registers, M0 stepped by 4 KiB. The waves issue these loads between two blocks' products,
+// where nothing else of the wave runs: with a 64-bit base, an LDS address and the wait states
+// worked out per load, two tiles took about 130 scalar instructions (2 x 2048 tokens, 28 heads:
+// forward 83.8 us, backward 279; 81.3 and 273 this way).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"  // m0 is clobbered on purpose
+QL_DEV uint32_t lds_addr(const char* p) {
+  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)p);
+}
 QL_DEV void dma_b128(const char* sbase, uint32_t voff, char* lds) {
-  const uint32_t m0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr_t)lds);
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1"
                :
-               : "v"(voff), "s"(sbase), "s"(m0)
+               : "v"(voff), "s"(sbase), "s"(lds_addr(lds))
                : "memory", "m0");
   QL_DMA_LOADED(lds);  // the 1 KiB this instruction fills: one span (tiles are 1-KiB aligned)
+}
+QL_DEV void dma_b128x4(const char* sbase, const uint32_t (&voff)[4], char* lds) {
+  asm volatile(
+      "s_mov_b32 m0, %5\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %4\n\t"
+      "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %4\n\t"
+      "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %4\n\t"
+      "s_add_u32 m0, m0, 0x1000\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %4"
+      :
+      : "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(sbase), "s"(lds_addr(lds))
+      : "memory", "m0", "scc");
+  for (int i = 0; i < 4; ++i) QL_DMA_LOADED(lds + i * 4096);
 }
 #pragma clang diagnostic pop
 
 struct TileDma {
-  uint32_t off;
-  int rsub, wave;
-  QL_DEV void init(int64_t ld, int wave_, int lane) {
+  const char* next;   // first row of the next tile
+  int64_t step;       // bytes from tile to tile
+  int64_t whole_end;  // tiles from row <= whole_end on are loaded by dma_b128x4
+  uint32_t voff[4];   // this lane's byte offset in load i, from the tile's first row
+  int wave;
+  // the tiles from row0 on, in turn
+  QL_DEV void init(const uint16_t* X, int64_t ld, int64_t row0, int64_t S, int wave_, int lane) {
     wave = wave_;
-    rsub = lane >> 4;
-    off = (uint32_t)rsub * (uint32_t)(ld * 2) +
-          (uint32_t)(swz_chunk(lane & 15, 4 * wave + rsub) * 16);
+    const int rsub = lane >> 4;
+    next = reinterpret_cast<const char*>(X + row0 * ld);
+    step = kRows * ld * 2;
+    whole_end = ld < (1 << 24) ? S - kRows : -1;  // a tile's offsets in 32 bits
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      voff[i] = (uint32_t)(16 * i + 4 * wave + rsub) * (uint32_t)(ld * 2) +
+                (uint32_t)(swz_chunk(lane & 15, 4 * wave + rsub) * 16);
   }
   QL_DEV void issue(const uint16_t* __restrict__ X, int64_t ld, int64_t row0, int64_t S,
-                    char* __restrict__ tile) const {
-    const int lane = threadIdx.x & 63;
-    if (row0 + kRows <= S) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int p = 4 * i + wave;
-        const char* base = reinterpret_cast<const char*>(X + (row0 + 4 * p) * ld);
-        dma_b128(base, off, tile + p * 1024);
-      }
+                    char* __restrict__ tile) {
+    if (row0 <= whole_end) {
+      dma_b128x4(next, voff, tile + wave * 1024);
     } else {
+      const int lane = threadIdx.x & 63, rsub = lane >> 4;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int p = 4 * i + wave;
@@ -212,6 +233,7 @@ struct TileDma {
         dma_b128(base, o, tile + p * 1024);
       }
     }
+    next += step;
   }
 };
 
@@ -253,9 +275,9 @@ struct AttnShape {
 // w owns query rows 32 w .. +31. Per 64-key block:
 //   S^T = K Q^T     K fragments from LDS, Q fragments in registers for the whole loop; a lane
 //                   owns one query column (lane % 16) and 4 keys per 16-key tile
-//   online softmax  per lane: block max over the lane's 16 keys plus two cross-lane steps, lazy
-//                   rescaling of O (only when the max rises by more than kTau), the row sum
-//                   kept per lane and combined once at the end
+//   online softmax  per lane: block max over the lane's 16 keys, lazy rescaling of O (only when
+//                   the max rises by more than kTau; two cross-lane steps then make the
+//                   column's max), the row sum kept per lane and combined once at the end
 //   O^T += V^T P^T  V^T fragments by transposing reads, P^T straight from registers
 template <int DT>
 struct FwdState {
@@ -270,7 +292,7 @@ struct FwdState {
 template <int DT>
 QL_DEV void fwd_block(FwdState<DT>& st, const char* __restrict__ kl, const char* __restrict__ vl,
                       char* __restrict__ kn, char* __restrict__ vn, bool issue,
-                      const TileDma& kdma, const TileDma& vdma, const uint16_t* __restrict__ kbase,
+                      TileDma& kdma, TileDma& vdma, const uint16_t* __restrict__ kbase,
                       const uint16_t* __restrict__ vbase, int64_t ks_s, int64_t vs_s, int64_t key0,
                       int64_t q0, int64_t S, float sl2, int lane) {
   const int fr = lane & 15, fq = lane >> 4;
@@ -302,7 +324,7 @@ QL_DEV void fwd_block(FwdState<DT>& st, const char* __restrict__ kl, const char*
   }
   __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
   __builtin_amdgcn_sched_barrier(0);
-  // mask keys after the query row or past the end; block max per query column
+  // mask keys after the query row or past the end; block max of the lane's keys per column
   const bool need_mask = key0 + kRows - 1 > q0 || key0 + kRows > S;
   float bm[2];
 #pragma unroll
@@ -322,14 +344,16 @@ QL_DEV void fwd_block(FwdState<DT>& st, const char* __restrict__ kl, const char*
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
       for (int e = 0; e < 4; ++e) mx = fmaxf(mx, s[qt][kt][e]);
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     bm[qt] = mx * sl2;
   }
+  // Some lane's keys raise its column's max by more than kTau exactly when the column's max
+  // does: the two cross-lane steps that make the column's max run only then.
   const bool raise = bm[0] > st.m[0] + kTau || bm[1] > st.m[1] + kTau;
   if (__builtin_amdgcn_ballot_w64(raise)) {
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt) {
+      bm[qt] = fmaxf(bm[qt], __shfl_xor(bm[qt], 16, 64));
+      bm[qt] = fmaxf(bm[qt], __shfl_xor(bm[qt], 32, 64));
       const float mn = fmaxf(st.m[qt], bm[qt]);
       const float alpha = __builtin_amdgcn_exp2f(st.m[qt] - mn);  // m = -inf: alpha = 0
       st.l[qt] *= alpha;
@@ -338,31 +362,44 @@ QL_DEV void fwd_block(FwdState<DT>& st, const char* __restrict__ kl, const char*
       st.m[qt] = mn;
     }
   }
-  uint4 pf[2][2];  // [ks][qt]
+  // P of keys 32 ks .. +31, packed as the B operand of the products with V
+  float rs[2] = {0.f, 0.f};
+  auto probs = [&](int ks, uint4 (&pf)[2]) {
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
-    const float nm = -st.m[qt];
-    float rs = 0.f;
+    for (int qt = 0; qt < 2; ++qt) {
+      const float nm = -st.m[qt];
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
+      for (int kt = 2 * ks; kt < 2 * ks + 2; ++kt)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[qt][kt][e], sl2, nm));
-        s[qt][kt][e] = p;
-        rs += p;
-      }
-    st.l[qt] += rs;
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) pf[ks][qt] = pack_pair<DT>(s[qt][2 * ks], s[qt][2 * ks + 1]);
-  }
-#pragma unroll
-  for (int ks = 0; ks < 2; ++ks)
+        for (int e = 0; e < 4; ++e) {
+          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[qt][kt][e], sl2, nm));
+          s[qt][kt][e] = p;
+          rs[qt] += p;
+        }
+      pf[qt] = pack_pair<DT>(s[qt][2 * ks], s[qt][2 * ks + 1]);
+    }
+  };
+  auto products = [&](int ks, const uint4 (&pf)[2]) {
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) {
       const uint4 vf = frag_tr(vl, 32 * ks, 16 * dt, fq, fr);
 #pragma unroll
-      for (int qt = 0; qt < 2; ++qt) st.o[qt][dt] = mfma<DT>(vf, pf[ks][qt], st.o[qt][dt]);
+      for (int qt = 0; qt < 2; ++qt) st.o[qt][dt] = mfma<DT>(vf, pf[qt], st.o[qt][dt]);
     }
+  };
+  // In two halves of 32 keys, the second half's exponentials beside the first half's products:
+  // one wave's exponentials and products take about as long as each other, and the two waves of
+  // a SIMD do not interleave them by themselves (2 x 2048 tokens, 28 heads: 86.8 us in one piece,
+  // 82.8 in halves; a fixed interleaving by schedule groups 85.6).
+  uint4 p0[2], p1[2];
+  probs(0, p0);
+  __builtin_amdgcn_sched_barrier(0);
+  probs(1, p1);
+#pragma unroll
+  for (int qt = 0; qt < 2; ++qt) st.l[qt] += rs[qt];
+  products(0, p0);
+  __builtin_amdgcn_sched_barrier(0);
+  products(1, p1);
 }
 
 template <int DT>
@@ -406,8 +443,8 @@ void attn_fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict_
   const int nkv = (int)((kv_end + kRows - 1) / kRows);
 
   TileDma kdma, vdma;
-  kdma.init(sh.ks_s, wave, lane);
-  vdma.init(sh.vs_s, wave, lane);
+  kdma.init(kbase, sh.ks_s, 0, S, wave, lane);
+  vdma.init(vbase, sh.vs_s, 0, S, wave, lane);
   kdma.issue(kbase, sh.ks_s, 0, S, smem);
   vdma.issue(vbase, sh.vs_s, 0, S, smem + kTileBytes);
   wait_vm_visible();  // the q fragments
@@ -473,7 +510,7 @@ struct DkdvState {
 
 template <int DT>
 QL_DEV void dkdv_block(DkdvState<DT>& st, const char* __restrict__ cur, char* __restrict__ nxt,
-                       bool issue, const TileDma& qdma, const TileDma& odma,
+                       bool issue, TileDma& qdma, TileDma& odma,
                        const uint16_t* __restrict__ qbase, const uint16_t* __restrict__ obase,
                        int64_t qs_s, int64_t os_s, int64_t qrow0, int64_t S, bool need_mask,
                        int kq_rel, int qlim, float sl2, int lane) {
@@ -592,8 +629,8 @@ void attn_bwd_dkdv(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ 
   const float* dl_row = delta + bh * S;
   const int n_qb = n_kblocks;  // 64-row query blocks
   TileDma qdma, odma;
-  qdma.init(sh.qs_s, wave, lane);
-  odma.init(sh.os_s, wave, lane);
+  qdma.init(qbase, sh.qs_s, (int64_t)kb * kRows, S, wave, lane);
+  odma.init(obase, sh.os_s, (int64_t)kb * kRows, S, wave, lane);
   // lse * log2e and Delta of a query block: thread t < 128 stages row t & 63 of one of them.
   // The load goes out before the block's math and the lse is scaled only where it is staged,
   // after that math, so no wave waits on the load's latency inside the block.
@@ -694,8 +731,8 @@ struct DqState {
 
 template <int DT>
 QL_DEV void dq_block(DqState<DT>& st, const char* __restrict__ kl, const char* __restrict__ vl,
-                     char* __restrict__ kn, char* __restrict__ vn, bool issue, const TileDma& kdma,
-                     const TileDma& vdma, const uint16_t* __restrict__ kbase,
+                     char* __restrict__ kn, char* __restrict__ vn, bool issue, TileDma& kdma,
+                     TileDma& vdma, const uint16_t* __restrict__ kbase,
                      const uint16_t* __restrict__ vbase, int64_t ks_s, int64_t vs_s, int64_t key0,
                      int64_t q0, int64_t S, float sl2, int lane) {
   const int fr = lane & 15, fq = lane >> 4;
@@ -851,8 +888,8 @@ void attn_bwd_dq(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
   const uint16_t* kbase = K + b * sh.ks_b + hk * sh.ks_h;
   const uint16_t* vbase = V + b * sh.vs_b + hk * sh.vs_h;
   TileDma kdma, vdma;
-  kdma.init(sh.ks_s, wave, lane);
-  vdma.init(sh.vs_s, wave, lane);
+  kdma.init(kbase, sh.ks_s, 0, S, wave, lane);
+  vdma.init(vbase, sh.vs_s, 0, S, wave, lane);
   kdma.issue(kbase, sh.ks_s, 0, S, smem);
   vdma.issue(vbase, sh.vs_s, 0, S, smem + kTileBytes);
   wait_vm_visible();  // the q and dO fragments and lse (Delta is computed above)
