@@ -47,7 +47,6 @@ constexpr int HD = 128;                         // head dim
 constexpr int kRows = 64;                       // rows per LDS tile / key block
 constexpr int kRowBytes = HD * 2;               // 256
 constexpr int kTileBytes = kRows * kRowBytes;   // 16 KiB
-constexpr int BQ = 128;                         // forward, dQ: query rows per workgroup
 constexpr int kThreads = 256;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
@@ -283,26 +282,26 @@ struct AttnShape {
 };
 
 // =============================================================================================
-// Forward. One workgroup per (b, hq, 128-row query block), the last blocks being the heaviest; wave
-// w owns query rows 32 w .. +31. Per 64-key block:
+// Forward. One workgroup per (b, hq, block of 64 QT query rows), the last blocks being the
+// heaviest; wave w owns query rows 16 QT w .. + 16 QT - 1. Per 64-key block:
 //   S^T = K Q^T     K fragments from LDS, Q fragments in registers for the whole loop; a lane
 //                   owns one query column (lane % 16) and 4 keys per 16-key tile
 //   online softmax  per lane: block max over the lane's 16 keys, lazy rescaling of O (only when
 //                   the max rises by more than kTau; two cross-lane steps then make the
 //                   column's max), the row sum kept per lane and combined once at the end
 //   O^T += V^T P^T  V^T fragments by transposing reads, P^T straight from registers
-template <int DT>
+template <int DT, int QT>
 struct FwdState {
-  uint4 qf[2][4];     // B operands: column q = 16 qt + lane % 16, d = 32 ds + 8 (lane / 16) ..
-  f32x4_t o[2][8];    // [qt][dt]: rows d = 16 dt + 4 (lane / 16) + e, column q
-  float m[2], l[2];
+  uint4 qf[QT][4];     // B operands: column q = 16 qt + lane % 16, d = 32 ds + 8 (lane / 16) ..
+  f32x4_t o[QT][8];    // [qt][dt]: rows d = 16 dt + 4 (lane / 16) + e, column q
+  float m[QT], l[QT];
 };
 
 // `kl`, `vl`: this block's K and V tiles; `kn`, `vn`: the other stage, which the next block's
 // DMA fills meanwhile (restrict keeps the compiler's wait-count pass from making these LDS
 // reads wait for that DMA).
-template <int DT>
-QL_DEV void fwd_block(FwdState<DT>& st, const char* __restrict__ kl, const char* __restrict__ vl,
+template <int DT, int QT>
+QL_DEV void fwd_block(FwdState<DT, QT>& st, const char* __restrict__ kl, const char* __restrict__ vl,
                       char* __restrict__ kn, char* __restrict__ vn, bool issue,
                       TileDma& kdma, TileDma& vdma, const uint16_t* __restrict__ kbase,
                       const uint16_t* __restrict__ vbase, int64_t ks_s, int64_t vs_s, int64_t key0,
@@ -312,10 +311,10 @@ QL_DEV void fwd_block(FwdState<DT>& st, const char* __restrict__ kl, const char*
     kdma.issue(kbase, ks_s, key0 + kRows, S, kn);
     vdma.issue(vbase, vs_s, key0 + kRows, S, vn);
   }
-  if (key0 > q0 + 31) return;  // every key of the block is after this wave's rows
-  f32x4_t s[2][4];
+  if (key0 > q0 + 16 * QT - 1) return;  // every key of the block is after this wave's rows
+  f32x4_t s[QT][4];
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt)
+  for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) s[qt][kt] = zero4();
   __builtin_amdgcn_sched_barrier(0);
@@ -325,22 +324,23 @@ QL_DEV void fwd_block(FwdState<DT>& st, const char* __restrict__ kl, const char*
     for (int kt = 0; kt < 4; ++kt) {
       const uint4 kf = frag_row(kl, 16 * kt + fr, ds, fq);
 #pragma unroll
-      for (int qt = 0; qt < 2; ++qt) s[qt][kt] = mfma<DT>(kf, st.qf[qt][ds], s[qt][kt]);
+      for (int qt = 0; qt < QT; ++qt) s[qt][kt] = mfma<DT>(kf, st.qf[qt][ds], s[qt][kt]);
     }
-  // 16 steps of 1 row read and 2 products; reads two steps ahead of their products
-  __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+  // 16 steps of 1 row read and QT products; reads 4 / QT steps ahead of their products
+  constexpr int kAhead = 4 / QT;
+  __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
 #pragma unroll
-  for (int i = 0; i < 14; ++i) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+  for (int i = 0; i < 16 - kAhead; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, QT, 0);
     __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
   }
-  __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+  __builtin_amdgcn_sched_group_barrier(0x008, QT * kAhead, 0);
   __builtin_amdgcn_sched_barrier(0);
   // mask keys after the query row or past the end; block max of the lane's keys per column
   const bool need_mask = key0 + kRows - 1 > q0 || key0 + kRows > S;
-  float bm[2];
+  float bm[QT];
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
+  for (int qt = 0; qt < QT; ++qt) {
     if (need_mask) {
       // key = key0 + 16 kt + 4 fq + e is kept iff 16 kt + e <= lim
       const int64_t q = q0 + 16 * qt + fr;
@@ -360,10 +360,11 @@ QL_DEV void fwd_block(FwdState<DT>& st, const char* __restrict__ kl, const char*
   }
   // Some lane's keys raise its column's max by more than kTau exactly when the column's max
   // does: the two cross-lane steps that make the column's max run only then.
-  const bool raise = bm[0] > st.m[0] + kTau || bm[1] > st.m[1] + kTau;
+  bool raise = bm[0] > st.m[0] + kTau;
+  if (QT == 2) raise = raise || bm[QT - 1] > st.m[QT - 1] + kTau;
   if (__builtin_amdgcn_ballot_w64(raise)) {
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt) {
+    for (int qt = 0; qt < QT; ++qt) {
       bm[qt] = fmaxf(bm[qt], __shfl_xor(bm[qt], 16, 64));
       bm[qt] = fmaxf(bm[qt], __shfl_xor(bm[qt], 32, 64));
       const float mn = fmaxf(st.m[qt], bm[qt]);
@@ -375,10 +376,10 @@ QL_DEV void fwd_block(FwdState<DT>& st, const char* __restrict__ kl, const char*
     }
   }
   // P of keys 32 ks .. +31, packed as the B operand of the products with V
-  float rs[2] = {0.f, 0.f};
-  auto probs = [&](int ks, uint4 (&pf)[2]) {
+  float rs[QT] = {};
+  auto probs = [&](int ks, uint4 (&pf)[QT]) {
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt) {
+    for (int qt = 0; qt < QT; ++qt) {
       const float nm = -st.m[qt];
 #pragma unroll
       for (int kt = 2 * ks; kt < 2 * ks + 2; ++kt)
@@ -391,36 +392,37 @@ QL_DEV void fwd_block(FwdState<DT>& st, const char* __restrict__ kl, const char*
       pf[qt] = pack_pair<DT>(s[qt][2 * ks], s[qt][2 * ks + 1]);
     }
   };
-  auto products = [&](int ks, const uint4 (&pf)[2]) {
+  auto products = [&](int ks, const uint4 (&pf)[QT]) {
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) {
       const uint4 vf = frag_tr(vl, 32 * ks, 16 * dt, fq, fr);
 #pragma unroll
-      for (int qt = 0; qt < 2; ++qt) st.o[qt][dt] = mfma<DT>(vf, pf[qt], st.o[qt][dt]);
+      for (int qt = 0; qt < QT; ++qt) st.o[qt][dt] = mfma<DT>(vf, pf[qt], st.o[qt][dt]);
     }
   };
   // In two halves of 32 keys, the second half's exponentials beside the first half's products:
   // one wave's exponentials and products take about as long as each other, and the two waves of
   // a SIMD do not interleave them by themselves (2 x 2048 tokens, 28 heads: 86.8 us in one piece,
   // 82.8 in halves; a fixed interleaving by schedule groups 85.6).
-  uint4 p0[2], p1[2];
+  uint4 p0[QT], p1[QT];
   probs(0, p0);
   __builtin_amdgcn_sched_barrier(0);
   probs(1, p1);
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) st.l[qt] += rs[qt];
+  for (int qt = 0; qt < QT; ++qt) st.l[qt] += rs[qt];
   products(0, p0);
   __builtin_amdgcn_sched_barrier(0);
   products(1, p1);
 }
 
-template <int DT>
+template <int DT, int QT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
                      const uint16_t* __restrict__ V, uint16_t* __restrict__ O,
                      float* __restrict__ lse, AttnShape sh, int n_qblocks) {
   __shared__ __attribute__((aligned(1024))) char smem[4 * kTileBytes];  // [stage][K, V]
   QL_DMA_BEGIN();
+  constexpr int BQ = 64 * QT;
   const int64_t BH = sh.B * sh.HQ;
   const unsigned item = work_item(blockIdx.x, gridDim.x);
   const int qb = n_qblocks - 1 - (int)(item / BH);  // the last blocks are the heaviest
@@ -431,15 +433,15 @@ void attn_fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict_
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int fr = lane & 15, fq = lane >> 4;
-  const int64_t q0 = (int64_t)qb * BQ + 32 * wave;  // this wave's first query row
+  const int64_t q0 = (int64_t)qb * BQ + 16 * QT * wave;  // this wave's first query row
 
   const uint16_t* qbase = Q + b * sh.qs_b + hq * sh.qs_h;
   const uint16_t* kbase = K + b * sh.ks_b + hk * sh.ks_h;
   const uint16_t* vbase = V + b * sh.vs_b + hk * sh.vs_h;
 
-  FwdState<DT> st;
+  FwdState<DT, QT> st;
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
+  for (int qt = 0; qt < QT; ++qt) {
     const int64_t q = q0 + 16 * qt + fr;
     const int64_t qc = q < S ? q : S - 1;
 #pragma unroll
@@ -467,14 +469,14 @@ void attn_fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict_
     wait_all_barrier();
     char* cur = smem + (j & 1) * 2 * kTileBytes;
     char* nxt = smem + ((j + 1) & 1) * 2 * kTileBytes;
-    fwd_block<DT>(st, cur, cur + kTileBytes, nxt, nxt + kTileBytes, j + 1 < nkv, kdma, vdma,
+    fwd_block<DT, QT>(st, cur, cur + kTileBytes, nxt, nxt + kTileBytes, j + 1 < nkv, kdma, vdma,
                   kbase, vbase, sh.ks_s, sh.vs_s, (int64_t)j * kRows, q0, S, sl2, lane);
   }
 
   // O = O^T / l, lse = (m + log2 l) ln 2 (natural log of sum exp(scale * s))
   uint16_t* obase = O + b * sh.os_b + hq * sh.os_h;
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
+  for (int qt = 0; qt < QT; ++qt) {
     float l = st.l[qt];
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
@@ -731,20 +733,20 @@ __global__ __launch_bounds__(256) void attn_bwd_reduce(const uint16_t* __restric
   Vec8<DT>::store(dV + o, av);
 }
 
-// ---- dQ: one workgroup per (b, hq, 128-row query block); wave w owns rows
-// 32 w .. +31. Per 64-key block, in two 32-key halves:
+// ---- dQ: one workgroup per (b, hq, block of 64 QT query rows); wave w owns rows 16 QT w ..
+// + 16 QT - 1. Per 64-key block, in two 32-key halves:
 //   S^T = K Q^T, dP^T = V dO^T    K, V row fragments from LDS; Q, dO fragments in registers
 //   dS^T = P^T (dP^T - Delta)
 //   dQ^T += K^T dS^T               K^T by transposing reads; dS^T from registers
-template <int DT>
+template <int DT, int QT>
 struct DqState {
-  uint4 qf[2][4], df[2][4];  // B operands: column q = 16 qt + lane % 16, d = 32 ds + 8 (lane/16)
-  f32x4_t dq[2][8];          // [qt][dt]: rows d = 16 dt + 4 (lane / 16) + e, column q
-  float l2[2], dl[2];        // lse * log2e and Delta of the lane's query columns
+  uint4 qf[QT][4], df[QT][4];  // B operands: column q = 16 qt + lane % 16, d = 32 ds + 8 (lane/16)
+  f32x4_t dq[QT][8];          // [qt][dt]: rows d = 16 dt + 4 (lane / 16) + e, column q
+  float l2[QT], dl[QT];        // lse * log2e and Delta of the lane's query columns
 };
 
-template <int DT>
-QL_DEV void dq_block(DqState<DT>& st, const char* __restrict__ kl, const char* __restrict__ vl,
+template <int DT, int QT>
+QL_DEV void dq_block(DqState<DT, QT>& st, const char* __restrict__ kl, const char* __restrict__ vl,
                      char* __restrict__ kn, char* __restrict__ vn, bool issue, TileDma& kdma,
                      TileDma& vdma, const uint16_t* __restrict__ kbase,
                      const uint16_t* __restrict__ vbase, int64_t ks_s, int64_t vs_s, int64_t key0,
@@ -754,16 +756,16 @@ QL_DEV void dq_block(DqState<DT>& st, const char* __restrict__ kl, const char* _
     kdma.issue(kbase, ks_s, key0 + kRows, S, kn);
     vdma.issue(vbase, vs_s, key0 + kRows, S, vn);
   }
-  if (key0 > q0 + 31) return;
+  if (key0 > q0 + 16 * QT - 1) return;
   const bool need_mask = key0 + kRows - 1 > q0 || key0 + kRows > S;
   // key - q = kq_rel + 32 h + 16 kk + e - 16 qt; keys at or past the end: 32 h + 16 kk + e >= klim
   const int kq_rel = clamp_rel(key0 + 4 * fq - (q0 + fr));
   const int klim = clamp_rel(S - key0 - 4 * fq);
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    f32x4_t sp[2][2], dp[2][2];  // [qt][kk]: rows key 32 h + 16 kk + 4 (lane/16) + e, column q
+    f32x4_t sp[QT][2], dp[QT][2];  // [qt][kk]: rows key 32 h + 16 kk + 4 (lane/16) + e, column q
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt)
+    for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) sp[qt][kk] = dp[qt][kk] = zero4();
     __builtin_amdgcn_sched_barrier(0);
@@ -775,22 +777,22 @@ QL_DEV void dq_block(DqState<DT>& st, const char* __restrict__ kl, const char* _
         const uint4 ka = frag_row(kl, row, ds, fq);
         const uint4 va = frag_row(vl, row, ds, fq);
 #pragma unroll
-        for (int qt = 0; qt < 2; ++qt) {
+        for (int qt = 0; qt < QT; ++qt) {
           sp[qt][kk] = mfma<DT>(ka, st.qf[qt][ds], sp[qt][kk]);
           dp[qt][kk] = mfma<DT>(va, st.df[qt][ds], dp[qt][kk]);
         }
       }
-    // 8 steps of 2 row reads and 4 products; reads two steps ahead of their products
+    // 8 steps of 2 row reads and 2 QT products; reads two steps ahead of their products
     __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
     for (int i = 0; i < 6; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 2 * QT, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 4 * QT, 0);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt)
+    for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -798,7 +800,7 @@ QL_DEV void dq_block(DqState<DT>& st, const char* __restrict__ kl, const char* _
           sp[qt][kk][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sp[qt][kk][e], sl2, -st.l2[qt]));
     if (__builtin_expect(need_mask, 0)) {  // wave-uniform: the diagonal and end blocks only
 #pragma unroll
-      for (int qt = 0; qt < 2; ++qt)
+      for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -807,9 +809,9 @@ QL_DEV void dq_block(DqState<DT>& st, const char* __restrict__ kl, const char* _
             if (kq_rel + rel - 16 * qt > 0 || rel >= klim) sp[qt][kk][e] = 0.f;
           }
     }
-    uint4 sb[2];
+    uint4 sb[QT];
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt) {
+    for (int qt = 0; qt < QT; ++qt) {
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -821,21 +823,21 @@ QL_DEV void dq_block(DqState<DT>& st, const char* __restrict__ kl, const char* _
     for (int dt = 0; dt < 8; ++dt) {
       const uint4 ka = frag_tr(kl, 32 * h, 16 * dt, fq, fr);
 #pragma unroll
-      for (int qt = 0; qt < 2; ++qt) st.dq[qt][dt] = mfma<DT>(ka, sb[qt], st.dq[qt][dt]);
+      for (int qt = 0; qt < QT; ++qt) st.dq[qt][dt] = mfma<DT>(ka, sb[qt], st.dq[qt][dt]);
     }
-    // 8 steps of 2 transposing reads and 2 products; reads two steps ahead
+    // 8 steps of 2 transposing reads and QT products; reads two steps ahead
     __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
     for (int i = 0; i < 6; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, QT, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 2 * QT, 0);
     __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-template <int DT>
+template <int DT, int QT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_bwd_dq(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
                  const uint16_t* __restrict__ V, const uint16_t* __restrict__ O,
@@ -844,6 +846,7 @@ void attn_bwd_dq(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
                  int n_qblocks) {
   __shared__ __attribute__((aligned(1024))) char smem[4 * kTileBytes];  // [stage][K, V]
   QL_DMA_BEGIN();
+  constexpr int BQ = 64 * QT;
   const int64_t BH = sh.B * sh.HQ;
   const unsigned item = work_item(blockIdx.x, gridDim.x);
   const int qb = n_qblocks - 1 - (int)(item / BH);  // the last blocks are the heaviest
@@ -854,15 +857,15 @@ void attn_bwd_dq(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int fr = lane & 15, fq = lane >> 4;
-  const int64_t q0 = (int64_t)qb * BQ + 32 * wave;
+  const int64_t q0 = (int64_t)qb * BQ + 16 * QT * wave;
   const float sl2 = sh.scale * kLog2e;
 
-  DqState<DT> st;
+  DqState<DT, QT> st;
   const uint16_t* qbase = Q + b * sh.qs_b + hq * sh.qs_h;
   const uint16_t* dobase = dO + b * sh.os_b + hq * sh.os_h;
   const uint16_t* obase = O + b * sh.os_b + hq * sh.os_h;
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
+  for (int qt = 0; qt < QT; ++qt) {
     const int64_t q = q0 + 16 * qt + fr;
     const int64_t qc = q < S ? q : S - 1;
     uint4 of[4];
@@ -912,12 +915,12 @@ void attn_bwd_dq(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
     wait_all_barrier();
     char* cur = smem + (j & 1) * 2 * kTileBytes;
     char* nxt = smem + ((j + 1) & 1) * 2 * kTileBytes;
-    dq_block<DT>(st, cur, cur + kTileBytes, nxt, nxt + kTileBytes, j + 1 < nkv, kdma, vdma,
+    dq_block<DT, QT>(st, cur, cur + kTileBytes, nxt, nxt + kTileBytes, j + 1 < nkv, kdma, vdma,
                  kbase, vbase, sh.ks_s, sh.vs_s, (int64_t)j * kRows, q0, S, sl2, lane);
   }
   uint16_t* dqb = dQ + b * sh.dq_b + hq * sh.dq_h;
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
+  for (int qt = 0; qt < QT; ++qt) {
     const int64_t q = q0 + 16 * qt + fr;
     if (q >= S) continue;
 #pragma unroll
@@ -928,6 +931,15 @@ void attn_bwd_dq(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
     }
   }
 }
+
+// Query tiles of 16 rows per wave in the forward and dQ kernels (64 QT query rows per
+// workgroup). 128 rows read K and V from LDS half as often per product; 64 rows make twice the
+// workgroups, each with about 0.6 of the latency per key block, and win while 128 rows leave a
+// compute unit fewer than its two workgroups. Forward / backward in us, 128 against 64 rows:
+//   84 items of 128 rows 13.1 / 39.2 : 9.9 / 34.7     216: 23.5 / 63.1 : 18.5 / 57.6
+//   256: 28.0 / 69.4 : 21.6 / 62.6   384 (S = 4096): 89.0 / 235 : 71.2 / 224
+//   448: 49.9 / 150 : 45.1 / 147     512: 50.5 / 160 : 49.9 / 163    576: 53.6 / 180 : 57.9 / 188
+int query_tiles(int64_t bh, int64_t S) { return bh * ((S + 127) / 128) < 2 * kUnits ? 1 : 2; }
 
 int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
 
@@ -956,18 +968,23 @@ extern "C" int qlora_attn_fwd(const void* q, const void* k, const void* v, void*
     if (st % 8) return QL_EALIGN;
   if (!ql_aligned(q, 16) || !ql_aligned(k, 16) || !ql_aligned(v, 16) || !ql_aligned(o, 16))
     return QL_EALIGN;
-  const int n_qblocks = (int)((S + BQ - 1) / BQ);
+  const int qt = query_tiles(B * HQ, S);
+  const int n_qblocks = (int)((S + 64 * qt - 1) / (64 * qt));
   const int64_t grid = B * HQ * n_qblocks;
   if (grid > INT32_MAX) return QL_EINVAL;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (dtype == QL_BF16)
-    hipLaunchKernelGGL((attn_fwd_kernel<QL_BF16>), dim3((unsigned)grid), dim3(kThreads), 0, s,
-                       (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o,
-                       lse, sh, n_qblocks);
-  else
-    hipLaunchKernelGGL((attn_fwd_kernel<QL_F16>), dim3((unsigned)grid), dim3(kThreads), 0, s,
-                       (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o,
-                       lse, sh, n_qblocks);
+#define QL_ATTN_FWD(DTC, QTC)                                                                     \
+  hipLaunchKernelGGL((attn_fwd_kernel<DTC, QTC>), dim3((unsigned)grid), dim3(kThreads), 0, s,     \
+                     (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o,    \
+                     lse, sh, n_qblocks)
+  if (dtype == QL_BF16) {
+    if (qt == 2) QL_ATTN_FWD(QL_BF16, 2);
+    else QL_ATTN_FWD(QL_BF16, 1);
+  } else {
+    if (qt == 2) QL_ATTN_FWD(QL_F16, 2);
+    else QL_ATTN_FWD(QL_F16, 1);
+  }
+#undef QL_ATTN_FWD
   return ql_launch_status();
 }
 
@@ -1022,16 +1039,20 @@ extern "C" int qlora_attn_bwd(const void* q, const void* k, const void* v, const
     pv = reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(pk) + part_bytes);
   }
   const int n_kblocks = (int)((S + kRows - 1) / kRows);
-  const int n_qblocks = (int)((S + BQ - 1) / BQ);
+  const int qt = query_tiles(B * HQ, S);
+  const int n_qblocks = (int)((S + 64 * qt - 1) / (64 * qt));
   if (B * HQ * n_kblocks > INT32_MAX || B * HQ * n_qblocks > INT32_MAX ||
       (B * HK * S * 16 + 255) / 256 > INT32_MAX)
     return QL_EINVAL;
+#define QL_ATTN_DQ(DTC, QTC)                                                                      \
+  hipLaunchKernelGGL((attn_bwd_dq<DTC, QTC>), dim3((unsigned)(B * HQ * n_qblocks)),               \
+                     dim3(kThreads), 0, s, (const uint16_t*)q, (const uint16_t*)k,                \
+                     (const uint16_t*)v, (const uint16_t*)o, (const uint16_t*)d_o, lse, delta,    \
+                     (uint16_t*)dq, sh, n_qblocks)
 #define QL_ATTN_BWD(DTC)                                                                          \
   do {                                                                                            \
-    hipLaunchKernelGGL((attn_bwd_dq<DTC>), dim3((unsigned)(B * HQ * n_qblocks)), dim3(kThreads),  \
-                       0, s, (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v,          \
-                       (const uint16_t*)o, (const uint16_t*)d_o, lse, delta, (uint16_t*)dq, sh,   \
-                       n_qblocks);                                                                \
+    if (qt == 2) QL_ATTN_DQ(DTC, 2);                                                              \
+    else QL_ATTN_DQ(DTC, 1);                                                                      \
     hipLaunchKernelGGL((attn_bwd_dkdv<DTC>), dim3((unsigned)(B * HQ * n_kblocks)), dim3(kThreads), \
                        0, s, (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v,          \
                        (const uint16_t*)d_o, lse, delta, (uint16_t*)dk, (uint16_t*)dv, pk, pv,    \
@@ -1043,6 +1064,7 @@ extern "C" int qlora_attn_bwd(const void* q, const void* k, const void* v, const
   if (dtype == QL_BF16) QL_ATTN_BWD(QL_BF16);
   else QL_ATTN_BWD(QL_F16);
 #undef QL_ATTN_BWD
+#undef QL_ATTN_DQ
   return ql_launch_status();
 }
 
