@@ -31,6 +31,8 @@
 //    with one barrier per block.
 //  - 4 waves per workgroup and at most 256 registers per lane, so two workgroups share a CU.
 // Head dim 128; any sequence length (rows and keys past the end are masked and clamped).
+#include <type_traits>
+
 #include "ql_vec.h"
 
 namespace {
@@ -219,7 +221,9 @@ struct TileDma {
     if (row0 <= whole_end) {
       dma_b128x4(next, voff, tile + wave * 1024);
     } else {
-      const int lane = threadIdx.x & 63, rsub = lane >> 4;
+      int lane = threadIdx.x & 63;
+      asm volatile("" : "+v"(lane));  // worked out here, not kept in registers by every block
+      const int rsub = lane >> 4;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int p = 4 * i + wave;
@@ -523,12 +527,17 @@ struct DkdvState {
   f32x4_t dv[8], dk[8];    // [dt]: rows d = 16 dt + 4 (lane / 16) + e, column key
 };
 
-template <int DT>
+// The four products of a block one after the other, each beside the element work that the next
+// needs: S; dP beside P = exp2(S - lse); dV += P^T dO beside dS = P (dP - Delta); dK += dS^T Q.
+// (S and dP together, then all element work, then dV and dK together: 157.7 us at 2 x 2048
+// tokens and 28 heads, 31.0 at 3 x 777 and 12, 17.3 at 333 and 28; this way 154.5, 30.3, 16.7.)
+// Mask: the block holds keys after a query row, or rows past the end.
+template <int DT, bool Mask>
 QL_DEV void dkdv_block(DkdvState<DT>& st, const char* __restrict__ cur, char* __restrict__ nxt,
                        bool issue, TileDma& qdma, TileDma& odma,
                        const uint16_t* __restrict__ qbase, const uint16_t* __restrict__ obase,
-                       int64_t qs_s, int64_t os_s, int64_t qrow0, int64_t S, bool need_mask,
-                       int kq_rel, int qlim, float sl2, int lane) {
+                       int64_t qs_s, int64_t os_s, int64_t qrow0, int64_t S, int kq_rel, int qlim,
+                       float sl2, int lane) {
   const int fr = lane & 15, fq = lane >> 4;
   if (issue) {
     qdma.issue(qbase, qs_s, qrow0 + kRows, S, nxt);
@@ -541,32 +550,41 @@ QL_DEV void dkdv_block(DkdvState<DT>& st, const char* __restrict__ cur, char* __
   f32x4_t sp[4], dp[4];  // [qt]: rows q = 16 qt + 4 (lane / 16) + e, column key
 #pragma unroll
   for (int qt = 0; qt < 4; ++qt) sp[qt] = dp[qt] = zero4();
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int ds = 0; ds < 4; ++ds)
 #pragma unroll
-    for (int qt = 0; qt < 4; ++qt) {
-      const int row = 16 * qt + fr;
-      sp[qt] = mfma<DT>(frag_row(q_l, row, ds, fq), st.kf[ds], sp[qt]);
-      dp[qt] = mfma<DT>(frag_row(do_l, row, ds, fq), st.vf[ds], dp[qt]);
-    }
+    for (int qt = 0; qt < 4; ++qt)
+      sp[qt] = mfma<DT>(frag_row(q_l, 16 * qt + fr, ds, fq), st.kf[ds], sp[qt]);
+  // 16 steps of 1 row read and 1 product; reads four steps ahead of their products
+  __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+  for (int i = 0; i < 12; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int qt = 0; qt < 4; ++qt) {
     const float4 l4 = *reinterpret_cast<const float4*>(lse2 + 16 * qt + 4 * fq);
     const float lv[4] = {l4.x, l4.y, l4.z, l4.w};
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
+    for (int e = 0; e < 4; ++e) {
       sp[qt][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sp[qt][e], sl2, -lv[e]));
+      // key - q = kq_rel - 16 qt - e; rows at or past the end: 16 qt + e >= qlim
+      if (Mask && (kq_rel - 16 * qt - e > 0 || 16 * qt + e >= qlim)) sp[qt][e] = 0.f;
+    }
   }
-  // Only the diagonal block and a block past the end have masked entries: a wave-uniform
-  // branch, so the other blocks skip the tests. key - q = kq_rel - 16 qt - e; rows at or past
-  // the end: 16 qt + e >= qlim.
-  if (__builtin_expect(need_mask, 0)) {
+  uint4 pb[2], sb[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) pb[ks] = pack_pair<DT>(sp[2 * ks], sp[2 * ks + 1]);
+#pragma unroll
+  for (int ds = 0; ds < 4; ++ds)
 #pragma unroll
     for (int qt = 0; qt < 4; ++qt)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (kq_rel - 16 * qt - e > 0 || 16 * qt + e >= qlim) sp[qt][e] = 0.f;
-  }
+      dp[qt] = mfma<DT>(frag_row(do_l, 16 * qt + fr, ds, fq), st.vf[ds], dp[qt]);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int qt = 0; qt < 4; ++qt) {
     const float4 d4 = *reinterpret_cast<const float4*>(dlt + 16 * qt + 4 * fq);
@@ -574,28 +592,23 @@ QL_DEV void dkdv_block(DkdvState<DT>& st, const char* __restrict__ cur, char* __
 #pragma unroll
     for (int e = 0; e < 4; ++e) dp[qt][e] = sp[qt][e] * (dp[qt][e] - dv[e]);
   }
-  uint4 pb[2], sb[2];
 #pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-    pb[ks] = pack_pair<DT>(sp[2 * ks], sp[2 * ks + 1]);
-    sb[ks] = pack_pair<DT>(dp[2 * ks], dp[2 * ks + 1]);
-  }
+  for (int ks = 0; ks < 2; ++ks) sb[ks] = pack_pair<DT>(dp[2 * ks], dp[2 * ks + 1]);
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    st.dv[i & 7] =
+        mfma<DT>(frag_tr(do_l, 32 * (i >> 3), 16 * (i & 7), fq, fr), pb[i >> 3], st.dv[i & 7]);
   __builtin_amdgcn_sched_barrier(0);
-  // 16 steps (ks, dt) of 4 transposing reads and 2 products. The reads run two steps ahead
-  // of their products, so a product waits on reads issued two steps earlier rather than on
-  // the latest one (left to itself the scheduler, short of registers, put each read right
-  // before its product and waited for it).
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int ks = i >> 3, dt = i & 7;
-    st.dv[dt] = mfma<DT>(frag_tr(do_l, 32 * ks, 16 * dt, fq, fr), pb[ks], st.dv[dt]);
-    st.dk[dt] = mfma<DT>(frag_tr(q_l, 32 * ks, 16 * dt, fq, fr), sb[ks], st.dk[dt]);
-  }
+  for (int i = 0; i < 16; ++i)
+    st.dk[i & 7] =
+        mfma<DT>(frag_tr(q_l, 32 * (i >> 3), 16 * (i & 7), fq, fr), sb[i >> 3], st.dk[i & 7]);
+  // 16 steps of 2 transposing reads and 1 product; reads four steps ahead
   __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
 #pragma unroll
-  for (int i = 0; i < 14; ++i) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+  for (int i = 0; i < 12; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
   }
   __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
   __builtin_amdgcn_sched_barrier(0);
@@ -663,7 +676,7 @@ void attn_bwd_dkdv(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ 
   odma.issue(obase, sh.os_s, (int64_t)kb * kRows, S, smem + kTileBytes);
   if (t < 128) stage_stat(smem, row_stat(kb));
   wait_vm_visible();  // the k and v fragments
-  for (int qb = kb; qb < n_qb; ++qb) {
+  auto step = [&](int qb, auto mask) {
     wait_all_barrier();
     const int it = qb - kb;
     char* cur = smem + (it & 1) * kBwdStage;
@@ -672,13 +685,17 @@ void attn_bwd_dkdv(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ 
     float stat = 0.f;
     if (more && t < 128) stat = row_stat(qb + 1);
     const int64_t qrow0 = (int64_t)qb * kRows;
-    const bool need_mask = qb == kb || qrow0 + kRows > S;
     const int kq_rel = clamp_rel(key0w + fr - (qrow0 + 4 * fq));
     const int qlim = clamp_rel(S - (qrow0 + 4 * fq));
-    dkdv_block<DT>(st, cur, nxt, more, qdma, odma, qbase, obase, sh.qs_s, sh.os_s, qrow0, S,
-                   need_mask, kq_rel, qlim, sl2, lane);
+    dkdv_block<DT, decltype(mask)::value>(st, cur, nxt, more, qdma, odma, qbase, obase, sh.qs_s,
+                                          sh.os_s, qrow0, S, kq_rel, qlim, sl2, lane);
     if (more && t < 128) stage_stat(nxt, stat);
-  }
+  };
+  // the diagonal block, those with every entry kept, and one past the end of the rows
+  step(kb, std::true_type{});
+  int qb = kb + 1;
+  for (; qb < (int)(S / kRows); ++qb) step(qb, std::false_type{});
+  if (qb < n_qb) step(qb, std::true_type{});
 
   const int64_t key = key0w + fr;
   if (key >= S) return;
