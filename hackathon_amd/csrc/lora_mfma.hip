@@ -2357,10 +2357,17 @@ extern "C" int qlora_lora_down(const void* X, int64_t ldx, const void* Y, int64_
 // least four chunks per wave in every split. Measured at 4096 rows (bf16, one adapter): K =
 // 18944 126-128 us split 4 against 135-136 us unsplit; at K = 3584 the split (then 4 x 14
 // chunks) cost 4-24 us more than it saved (the partials and their reduce), so it stays unsplit.
+// While the workgroups do not fill the chip once, a workgroup's time is its chunks' alone and a
+// split shortens it, down to three chunks (bf16, one adapter / three, us, unsplit : split so):
+//   M = 1001, K = 3584  22.6 / 52.9 : 11.8 / 21.7      M = 333   22.4 / 53.3 : 8.1 / 13.3
+//   M = 16, K = 4864    18.7 / 40.9 : 7.8 / 12.6       M = 2048, K = 896  8.7 / 18.3 : 8.2 / 13.9
+// Past one filling it costs: M = 1001, K = 3584 in 8 splits (504 workgroups) 10.8 / 22.8, in 16
+// 13.3 / 26.6.
 static int ql_dropout_down_splits(int64_t M, int64_t K) {
   const int64_t blocks = (M + 15) / 16, nch = K / 64;
   int s = 1;
   while (blocks * s < 1024 && nch / (2 * s) >= 4 * kDdWaves && s < 64) s *= 2;
+  while (blocks * 2 * s <= 256 && nch >= 3 * 2 * s && s < 64) s *= 2;
   return s;
 }
 
