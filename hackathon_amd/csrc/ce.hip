@@ -16,9 +16,15 @@
 // Second reads stay on chip: each thread keeps its first chunks of the row (the row's first
 // 64 KiB) in LDS for sweep 2, and the 64 KiB per workgroup hold the GPU at two rows per CU,
 // so the 512 rows in flight (156 MB at the Qwen2 vocabulary, 151936 x 2 B a row) stay inside
-// the 256 MB MALL and the rest of sweep 2 reads from there. Sweep 1 issues 4 chunk loads and
-// sweep 2 8 before their arithmetic. 8192 x 151936 bf16 on MI355X: 1.15 ms, against 1.45 ms
-// with four rows per CU and one chunk per step (the 1024 rows in flight spilled the MALL).
+// the 256 MB MALL and the rest of sweep 2 reads from there (1.15 ms for 8192 x 151936 bf16, against
+// 1.45 ms with four rows per CU: the 1024 rows in flight spilled the MALL). Both sweeps load 4
+// chunks, then do their arithmetic as one piece: one maximum, one rescaling, one test for small
+// exponents, the target's entry by itself. With a maximum and its index, a scaled exponential
+// and a 64-bit target test per element the vector ALU took as long as the memory (4096 x 151936
+// bf16 641 us, 512 x 151936 82.6, 1000 x 32000 47.4; now 594, 69, 35). 8 chunks at a time need
+// more than the 128 registers of four waves per SIMD: 690, 77, 47.
+#include <type_traits>
+
 #include "ql_vec.h"
 
 namespace {
@@ -56,8 +62,25 @@ QL_DEV RowStat shfl_stat(const RowStat& v, int off) {
   return r;
 }
 
+// v[j] = exp2f(v[j]). exp2f is v_exp_f32 except below -126, where it scales the argument up and
+// the (subnormal) result down, five more instructions per element. A wave without such an
+// element takes v_exp_f32 alone, with the same bits.
+template <int N>
+QL_DEV void exp2_chunk(float* v) {
+  float lo = v[0];
+#pragma unroll
+  for (int j = 1; j < N; ++j) lo = fminf(lo, v[j]);
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(lo < -126.f) == 0, 1)) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) v[j] = __builtin_amdgcn_exp2f(v[j]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < N; ++j) v[j] = exp2f(v[j]);
+  }
+}
+
 constexpr int kCacheBytes = 64 * 1024;  // LDS row cache per workgroup (dynamic)
-constexpr int kUnroll1 = 4, kUnroll2 = 8;  // chunk loads in flight per thread, sweeps 1 and 2
+constexpr int kUnroll = 4;  // chunk loads in flight per thread
 
 // VW = 8: 8-element chunks (V % 8 == 0, 16-B aligned rows), 16-bit ones cached in LDS;
 // VW = 1: one element per step, no cache.
@@ -72,7 +95,7 @@ __global__ __launch_bounds__(kThreads) void ce_rows_kernel(
   __shared__ float lse_sh;
   constexpr bool kCached = VW == 8 && DT != QL_F32;  // a 16-B chunk per 8 elements
   constexpr int64_t kCacheChunks = kCached ? kCacheBytes / 16 : 0;
-  constexpr int U1 = VW == 8 ? kUnroll1 : 1, U2 = VW == 8 ? kUnroll2 : 1;
+  constexpr int U = VW == 8 ? kUnroll : 1;
   const int64_t row = blockIdx.x;
   auto* z = logits + row * row_stride;
   const int64_t tgt = target[row];
@@ -99,40 +122,64 @@ __global__ __launch_bounds__(kThreads) void ce_rows_kernel(
   };
 
   RowStat st{-INFINITY, 0.f, 0.f, -INFINITY, 0};
-  auto absorb = [&](const float* v, int64_t c) {
-    float cm = v[0];
-    int cj = 0;
+  int64_t best_c = -1;  // the first chunk with this thread's maximum
+  // N chunks, c and every kThreads-th after it: one rescaling of the sums for all of them
+  auto absorb = [&](auto count, const float (*v)[VW], int64_t c) {
+    constexpr int N = decltype(count)::value;
+    float cm[N], gm = -INFINITY;
 #pragma unroll
-    for (int j = 1; j < VW; ++j)
-      if (v[j] > cm) { cm = v[j]; cj = j; }
-    if (cm > st.best) { st.best = cm; st.best_idx = c * VW + cj; }
-    const float m = fmaxf(st.m, cm);
-    const float alpha = (st.m == -INFINITY) ? 0.f : exp2f((st.m - m) * kLog2e);
-    float es = 0.f, et = 0.f;
+    for (int u = 0; u < N; ++u) {
+      cm[u] = v[u][0];
 #pragma unroll
-    for (int j = 0; j < VW; ++j) {
-      const float e = exp2f((v[j] - m) * kLog2e);
-      es += e;
-      et += e * v[j];
+      for (int j = 1; j < VW; ++j) cm[u] = fmaxf(cm[u], v[u][j]);
+      cm[u] = v[u][0] == v[u][0] ? cm[u] : v[u][0];  // one that starts with NaN is never the maximum
+      gm = fmaxf(gm, cm[u]);
     }
+    if (gm > st.best) {
+      st.best = gm;
+#pragma unroll
+      for (int u = N - 1; u >= 0; --u) best_c = cm[u] == gm ? c + u * kThreads : best_c;
+    }
+    const float m = fmaxf(st.m, gm);
+    const float alpha = (st.m == -INFINITY) ? 0.f : exp2f((st.m - m) * kLog2e);
+    float e[N * VW], es = 0.f, et = 0.f;
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+#pragma unroll
+      for (int j = 0; j < VW; ++j) e[u * VW + j] = (v[u][j] - m) * kLog2e;
+    exp2_chunk<N * VW>(e);
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+#pragma unroll
+      for (int j = 0; j < VW; ++j) {
+        es += e[u * VW + j];
+        et += e[u * VW + j] * v[u][j];
+      }
     st.s = st.s * alpha + es;
     st.t = st.t * alpha + et;
     st.m = m;
   };
-  // Sweep 1, in increasing chunk order per thread (the first maximum wins): U1 loads, then
+  // Sweep 1, in increasing chunk order per thread (the first maximum wins): U loads, then
   // their arithmetic; chunks below kCacheChunks are also kept in LDS for sweep 2.
   int64_t c0 = threadIdx.x;
-  for (; c0 + (U1 - 1) * kThreads < nchunk; c0 += U1 * kThreads) {
-    float v[U1][VW];
+  for (; c0 + (U - 1) * kThreads < nchunk; c0 += U * kThreads) {
+    float v[U][VW];
 #pragma unroll
-    for (int u = 0; u < U1; ++u) load_keep(c0 + u * kThreads, v[u]);
-#pragma unroll
-    for (int u = 0; u < U1; ++u) absorb(v[u], c0 + u * kThreads);
+    for (int u = 0; u < U; ++u) load_keep(c0 + u * kThreads, v[u]);
+    absorb(std::integral_constant<int, U>{}, v, c0);
   }
   for (int64_t c = c0; c < nchunk; c += kThreads) {
+    float v[1][VW];
+    load_keep(c, v[0]);
+    absorb(std::integral_constant<int, 1>{}, v, c);
+  }
+  if (best_c >= 0) {  // the first element of that chunk that holds it
     float v[VW];
-    load_keep(c, v);
-    absorb(v, c);
+    load(best_c, v);
+    int j = VW - 1;
+#pragma unroll
+    for (int i = VW - 2; i >= 0; --i) j = v[i] == st.best ? i : j;
+    st.best_idx = best_c * VW + j;
   }
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) merge(st, shfl_stat(st, off));
@@ -156,29 +203,39 @@ __global__ __launch_bounds__(kThreads) void ce_rows_kernel(
   __syncthreads();
   const float lse = lse_sh;
   const float gs = labelled ? (grad_scale_dev ? *grad_scale_dev : grad_scale) : 0.f;
-  auto emit = [&](float* v, int64_t c) {
+  auto emit = [&](auto count, float (*v)[VW], int64_t c) {
+    constexpr int N = decltype(count)::value;
 #pragma unroll
-    for (int j = 0; j < VW; ++j) {
-      const float onehot = (c * VW + j == tgt) ? 1.f : 0.f;
-      v[j] = (exp2f((v[j] - lse) * kLog2e) - onehot) * gs;
+    for (int u = 0; u < N; ++u)
+#pragma unroll
+      for (int j = 0; j < VW; ++j) v[u][j] = (v[u][j] - lse) * kLog2e;
+    exp2_chunk<N * VW>(v[0]);
+#pragma unroll
+    for (int u = 0; u < N; ++u, c += kThreads) {
+      const int64_t hot = tgt - c * VW;
+      if (hot >= 0 && hot < VW) {  // one thread of the row, once
+#pragma unroll
+        for (int j = 0; j < VW; ++j) v[u][j] = j == (int)hot ? v[u][j] - 1.f : v[u][j];
+      }
+#pragma unroll
+      for (int j = 0; j < VW; ++j) v[u][j] *= gs;
+      if constexpr (VW == 8) Vec8<DT>::store(z + 8 * c, v[u]);
+      else z[c] = Elem<DT>::from_f32(v[u][0]);
     }
-    if constexpr (VW == 8) Vec8<DT>::store(z + 8 * c, v);
-    else z[c] = Elem<DT>::from_f32(v[0]);
   };
-  // Sweep 2: every thread rewrites the chunks it read (its cached ones from LDS), U2 loads
+  // Sweep 2: every thread rewrites the chunks it read (its cached ones from LDS), U loads
   // ahead of their arithmetic.
   c0 = threadIdx.x;
-  for (; c0 + (U2 - 1) * kThreads < nchunk; c0 += U2 * kThreads) {
-    float v[U2][VW];
+  for (; c0 + (U - 1) * kThreads < nchunk; c0 += U * kThreads) {
+    float v[U][VW];
 #pragma unroll
-    for (int u = 0; u < U2; ++u) load(c0 + u * kThreads, v[u]);
-#pragma unroll
-    for (int u = 0; u < U2; ++u) emit(v[u], c0 + u * kThreads);
+    for (int u = 0; u < U; ++u) load(c0 + u * kThreads, v[u]);
+    emit(std::integral_constant<int, U>{}, v, c0);
   }
   for (int64_t c = c0; c < nchunk; c += kThreads) {
-    float v[VW];
-    load(c, v);
-    emit(v, c);
+    float v[1][VW];
+    load(c, v[0]);
+    emit(std::integral_constant<int, 1>{}, v, c);
   }
 }
 
