@@ -173,11 +173,11 @@ std::vector<Weight> weights(const py::sequence& s) {
   return out;
 }
 
-// Every W_g [n_g, K] into its rows of w (one launch for 2 to 4 weights that the group kernel
-// takes, else one each).
+// Every W_g [n_g, K] into its rows of w (one launch for up to 4 weights that the group kernel
+// takes, else one each; a lone weight takes it for its stores, which stay in the caches).
 void dequant(const Ctx& c, const std::vector<Weight>& ws, const Tensor& w) {
   ql_nf4_weight d[4];
-  bool group = ws.size() >= 2 && ws.size() <= 4;
+  bool group = ws.size() >= 1 && ws.size() <= 4;
   int64_t off = 0;
   std::vector<char*> outs;
   for (const auto& x : ws) {
@@ -203,7 +203,7 @@ void dequant(const Ctx& c, const std::vector<Weight>& ws, const Tensor& w) {
 // Every W_g^T [K, n_g] into its columns of wt.
 void dequant_t(const Ctx& c, const std::vector<Weight>& ws, const Tensor& wt) {
   ql_nf4_weight d[4];
-  bool group = ws.size() >= 2 && ws.size() <= 4 && wt.stride(0) % 8 == 0;
+  bool group = ws.size() >= 1 && ws.size() <= 4 && wt.stride(0) % 8 == 0;
   int64_t off = 0;
   std::vector<char*> outs;
   for (const auto& x : ws) {

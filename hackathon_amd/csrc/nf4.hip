@@ -27,23 +27,28 @@ constexpr int kThreads = 256;
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
+template <bool KEEP> QL_DEV void store16(u32x4 v, u32x4* p) {
+  if constexpr (KEEP) *p = v;
+  else __builtin_nontemporal_store(v, p);
+}
+
 template <int OUT_DT> struct Group8;  // 8 dequantised weights -> one vector store
 template <> struct Group8<QL_BF16> {
-  static QL_DEV void store(uint16_t* out, int64_t g, const float* w) {
+  template <bool KEEP> static QL_DEV void store(uint16_t* out, int64_t g, const float* w) {
     const u32x4 v = {pack_bf16x2(w[0], w[1]), pack_bf16x2(w[2], w[3]), pack_bf16x2(w[4], w[5]),
                      pack_bf16x2(w[6], w[7])};
-    __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(out) + g);
+    store16<KEEP>(v, reinterpret_cast<u32x4*>(out) + g);
   }
 };
 template <> struct Group8<QL_F16> {
-  static QL_DEV void store(uint16_t* out, int64_t g, const float* w) {
+  template <bool KEEP> static QL_DEV void store(uint16_t* out, int64_t g, const float* w) {
     const u32x4 v = {pack_f16x2(w[0], w[1]), pack_f16x2(w[2], w[3]), pack_f16x2(w[4], w[5]),
                      pack_f16x2(w[6], w[7])};
-    __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(out) + g);
+    store16<KEEP>(v, reinterpret_cast<u32x4*>(out) + g);
   }
 };
 template <> struct Group8<QL_F32> {
-  static QL_DEV void store(float* out, int64_t g, const float* w) {
+  template <bool KEEP> static QL_DEV void store(float* out, int64_t g, const float* w) {
     float4* o = reinterpret_cast<float4*>(out) + 2 * g;
     o[0] = make_float4(w[0], w[1], w[2], w[3]);
     o[1] = make_float4(w[4], w[5], w[6], w[7]);
@@ -74,7 +79,7 @@ QL_DEV float block_scale(int64_t blk, const uint8_t* __restrict__ absmax_q,
 
 // One workgroup's span of the vector path: groups tile * kThreads * UNROLL + [0, kThreads *
 // UNROLL) of one weight.
-template <int OUT_DT, bool NESTED, int UNROLL>
+template <int OUT_DT, bool NESTED, int UNROLL, bool KEEP>
 QL_DEV void dequant_vec_span(int64_t tile, const uint32_t* __restrict__ packed4, int64_t n_groups,
                              const uint8_t* __restrict__ absmax_q,
                              const float* __restrict__ absmax_f, const float* __restrict__ code2,
@@ -128,7 +133,7 @@ QL_DEV void dequant_vec_span(int64_t tile, const uint32_t* __restrict__ packed4,
       w[2 * b] = fp32_rounded(table[byte >> 4] * s);      // high nibble: the first weight
       w[2 * b + 1] = fp32_rounded(table[byte & 15u] * s);  // low nibble: the second
     }
-    Group8<OUT_DT>::store(out, g, w);
+    Group8<OUT_DT>::template store<KEEP>(out, g, w);
   }
 }
 
@@ -138,9 +143,9 @@ __global__ __launch_bounds__(kThreads) void nf4_dequant_vec(
     const float* __restrict__ absmax_f, const float* __restrict__ code2,
     const float* __restrict__ absmax2, float offset, int log2_bs, int log2_bs2,
     const float* __restrict__ nf4_table, typename Elem<OUT_DT>::T* __restrict__ out) {
-  dequant_vec_span<OUT_DT, NESTED, UNROLL>(blockIdx.x, packed4, n_groups, absmax_q, absmax_f,
-                                           code2, absmax2, offset, log2_bs, log2_bs2, nf4_table,
-                                           out);
+  dequant_vec_span<OUT_DT, NESTED, UNROLL, false>(blockIdx.x, packed4, n_groups, absmax_q,
+                                                  absmax_f, code2, absmax2, offset, log2_bs,
+                                                  log2_bs2, nf4_table, out);
 }
 
 // Several weights in one launch (the q/k/v or gate/up projections of a layer): one launch
@@ -175,11 +180,11 @@ QL_DEV DqItem pick_item(const DqGroup& grp, uint32_t bx) {
   return it;
 }
 
-template <int OUT_DT, bool NESTED, int UNROLL>
+template <int OUT_DT, bool NESTED, int UNROLL, bool KEEP>
 __global__ __launch_bounds__(kThreads) void nf4_dequant_vec_group(
     const DqGroup grp, const float* __restrict__ nf4_table) {
   const DqItem it = pick_item(grp, blockIdx.x);
-  dequant_vec_span<OUT_DT, NESTED, UNROLL>(
+  dequant_vec_span<OUT_DT, NESTED, UNROLL, KEEP>(
       blockIdx.x - it.tile_begin, reinterpret_cast<const uint32_t*>(it.packed), it.rows,
       it.absmax_q, it.absmax_f, it.code2, it.absmax2, it.offset, it.log2_bs, it.log2_bs2,
       nf4_table, static_cast<typename Elem<OUT_DT>::T*>(it.out));
@@ -224,7 +229,7 @@ constexpr int kTStride = 36;  // LDS words per k-row of the tile (32 used, 16-B 
 constexpr int kTInStride = 17;  // LDS words per packed input row (16 used)
 
 // One 64 x 128 tile (n-tile nt, k-tile kt) of the transposed dequantisation.
-template <int OUT_DT, bool NESTED>
+template <int OUT_DT, bool NESTED, bool KEEP>
 QL_DEV void dequant_t_tile(int64_t nt, int64_t kt, const uint8_t* __restrict__ packed,
                            int64_t rows, int64_t cols, const uint8_t* __restrict__ absmax_q,
                            const float* __restrict__ absmax_f, const float* __restrict__ code2,
@@ -289,7 +294,7 @@ QL_DEV void dequant_t_tile(int64_t nt, int64_t kt, const uint8_t* __restrict__ p
     const int kr = (threadIdx.x >> 3) + 32 * i;
     if (n < rows) {  // rows % 8 == 0: a 16-B chunk is entirely in or out
       const u32x4 v = *reinterpret_cast<const u32x4*>(&tile[kr * kTStride + 4 * c]);
-      __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(outT + (k0 + kr) * ld_out + n));
+      store16<KEEP>(v, reinterpret_cast<u32x4*>(outT + (k0 + kr) * ld_out + n));
     }
   }
 }
@@ -301,23 +306,23 @@ __global__ __launch_bounds__(kThreads) void nf4_dequant_t_kernel(
     const float* __restrict__ code2, const float* __restrict__ absmax2, float offset, int log2_bs,
     int log2_bs2, const float* __restrict__ nf4_table, uint16_t* __restrict__ outT,
     int64_t ld_out) {
-  dequant_t_tile<OUT_DT, NESTED>(blockIdx.x, blockIdx.y, packed, rows, cols, absmax_q, absmax_f,
-                                 code2, absmax2, offset, log2_bs, log2_bs2, nf4_table, outT,
-                                 ld_out);
+  dequant_t_tile<OUT_DT, NESTED, false>(blockIdx.x, blockIdx.y, packed, rows, cols, absmax_q,
+                                        absmax_f, code2, absmax2, offset, log2_bs, log2_bs2,
+                                        nf4_table, outT, ld_out);
 }
 
 // Grouped transposed dequantisation: weight i's n-tiles are x indices [tile_begin_i, ..) and
 // its output block starts at item.out (its column offset in the shared out_t); the k-tiles
 // (y) run to the widest weight and a narrower weight's surplus workgroups exit at once.
-template <int OUT_DT, bool NESTED>
+template <int OUT_DT, bool NESTED, bool KEEP>
 __global__ __launch_bounds__(kThreads) void nf4_dequant_t_group(
     const DqGroup grp, const float* __restrict__ nf4_table, int64_t ld_out) {
   const DqItem it = pick_item(grp, blockIdx.x);
   if ((int64_t)blockIdx.y * kTCols >= it.cols) return;  // whole workgroup, before any barrier
-  dequant_t_tile<OUT_DT, NESTED>(blockIdx.x - it.tile_begin, blockIdx.y, it.packed, it.rows,
-                                 it.cols, it.absmax_q, it.absmax_f, it.code2, it.absmax2,
-                                 it.offset, it.log2_bs, it.log2_bs2, nf4_table,
-                                 static_cast<uint16_t*>(it.out), ld_out);
+  dequant_t_tile<OUT_DT, NESTED, KEEP>(blockIdx.x - it.tile_begin, blockIdx.y, it.packed, it.rows,
+                                       it.cols, it.absmax_q, it.absmax_f, it.code2, it.absmax2,
+                                       it.offset, it.log2_bs, it.log2_bs2, nf4_table,
+                                       static_cast<uint16_t*>(it.out), ld_out);
 }
 
 int ilog2_exact(int64_t v) {  // log2 of a power of two, else -1
@@ -458,10 +463,25 @@ int group_item(const ql_nf4_weight& w, int nested, bool transposed, int64_t ld_o
   return QL_OK;
 }
 
+// The group entries write weights that the layer's own product reads next: up to 32 MiB, what the
+// eight 4-MiB L2 caches hold together, with ordinary stores, so that they are found there.
+// Dequantisation and product, us, nontemporal : ordinary (bf16; W then W^T):
+//   2 MB [1152, 896], 1001 rows    13.9 / 16.0 : 12.5 / 13.8
+//   24.5 MB [3584, 3584], 1001     43.4 / 45.6 : 38.7 / 40.6
+//   31.5 MB [4608, 3584], 333      36.4 / 35.7 : 30.2 / 34.7     1001  75.1 / 54.3 : 62.1 / 48.3
+//   52.5 MB [17920, 1536], 333     44.9 / 52.0 : 41.4 / 55.2
+//   98 MB [14336, 3584], 333       80.5 / 84.3 : 85.1 / 87.4
+constexpr int64_t kKeepBytes = int64_t(32) << 20;
+
 template <int OUT_DT, bool NESTED>
-void launch_group(const DqGroup& grp, uint32_t tiles, const float* table, hipStream_t s) {
-  hipLaunchKernelGGL((nf4_dequant_vec_group<OUT_DT, NESTED, 2>), dim3(tiles), dim3(kThreads), 0,
-                     s, grp, table);
+void launch_group(const DqGroup& grp, uint32_t tiles, bool keep, const float* table,
+                  hipStream_t s) {
+  if (keep)
+    hipLaunchKernelGGL((nf4_dequant_vec_group<OUT_DT, NESTED, 2, true>), dim3(tiles),
+                       dim3(kThreads), 0, s, grp, table);
+  else
+    hipLaunchKernelGGL((nf4_dequant_vec_group<OUT_DT, NESTED, 2, false>), dim3(tiles),
+                       dim3(kThreads), 0, s, grp, table);
 }
 
 }  // namespace
@@ -471,13 +491,14 @@ extern "C" int qlora_nf4_dequant_group(const ql_nf4_weight* weights, int count, 
                                        ql_stream_t stream) {
   if (count < 1 || count > kMaxGroup || !weights || !nf4_table) return QL_EINVAL;
   DqGroup grp{};
-  int64_t tiles = 0;
+  int64_t tiles = 0, bytes = 0;
   for (int i = 0; i < count; ++i) {
     DqItem it{};
     const int st = group_item(weights[i], nested, false, 0, &it);
     if (st != QL_OK) return st;
     if (it.rows == 0 || weights[i].rows == 0 || weights[i].cols == 0) continue;
     it.tile_begin = (uint32_t)tiles;
+    bytes += 16 * it.rows;
     tiles += (it.rows + kThreads * 2 - 1) / (kThreads * 2);
     if (tiles > INT32_MAX) return QL_ESHAPE;
     grp.item[grp.count++] = it;
@@ -485,9 +506,9 @@ extern "C" int qlora_nf4_dequant_group(const ql_nf4_weight* weights, int count, 
   if (grp.count == 0) return QL_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (nested) {
-    QL_DISPATCH_DTYPE(out_dtype, DT, launch_group<DT, true>(grp, (uint32_t)tiles, nf4_table, s));
+    QL_DISPATCH_DTYPE(out_dtype, DT, launch_group<DT, true>(grp, (uint32_t)tiles, bytes <= kKeepBytes, nf4_table, s));
   } else {
-    QL_DISPATCH_DTYPE(out_dtype, DT, launch_group<DT, false>(grp, (uint32_t)tiles, nf4_table, s));
+    QL_DISPATCH_DTYPE(out_dtype, DT, launch_group<DT, false>(grp, (uint32_t)tiles, bytes <= kKeepBytes, nf4_table, s));
   }
   return ql_launch_status();
 }
@@ -499,7 +520,7 @@ extern "C" int qlora_nf4_dequant_t_group(const ql_nf4_weight* weights, int count
   if (out_dtype != QL_BF16 && out_dtype != QL_F16) return QL_EDTYPE;
   if (ld_out % 8) return QL_ESHAPE;
   DqGroup grp{};
-  int64_t tiles = 0, max_cols = 0;
+  int64_t tiles = 0, max_cols = 0, bytes = 0;
   for (int i = 0; i < count; ++i) {
     DqItem it{};
     const int st = group_item(weights[i], nested, true, ld_out, &it);
@@ -509,19 +530,28 @@ extern "C" int qlora_nf4_dequant_t_group(const ql_nf4_weight* weights, int count
     tiles += (it.rows + kTRows - 1) / kTRows;
     if (tiles > INT32_MAX) return QL_ESHAPE;
     max_cols = it.cols > max_cols ? it.cols : max_cols;
+    bytes += 2 * it.rows * it.cols;
     grp.item[grp.count++] = it;
   }
   if (grp.count == 0) return QL_OK;
   if (max_cols / kTCols > 65535) return QL_ESHAPE;
   const dim3 grid((unsigned)tiles, (unsigned)(max_cols / kTCols));
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define QL_DQTG(DT, NST)                                                                      \
-  hipLaunchKernelGGL((nf4_dequant_t_group<DT, NST>), grid, dim3(kThreads), 0, s, grp, nf4_table, \
-                     ld_out)
+#define QL_DQTG(DT, NST)                                                                          \
+  do {                                                                                            \
+    if (bytes <= kKeepBytes)                                                                      \
+      hipLaunchKernelGGL((nf4_dequant_t_group<DT, NST, true>), grid, dim3(kThreads), 0, s, grp,   \
+                         nf4_table, ld_out);                                                      \
+    else                                                                                          \
+      hipLaunchKernelGGL((nf4_dequant_t_group<DT, NST, false>), grid, dim3(kThreads), 0, s, grp,  \
+                         nf4_table, ld_out);                                                      \
+  } while (0)
   if (out_dtype == QL_BF16) {
-    if (nested) QL_DQTG(QL_BF16, true); else QL_DQTG(QL_BF16, false);
+    if (nested) QL_DQTG(QL_BF16, true);
+    else QL_DQTG(QL_BF16, false);
   } else {
-    if (nested) QL_DQTG(QL_F16, true); else QL_DQTG(QL_F16, false);
+    if (nested) QL_DQTG(QL_F16, true);
+    else QL_DQTG(QL_F16, false);
   }
 #undef QL_DQTG
   return ql_launch_status();
