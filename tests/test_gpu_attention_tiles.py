@@ -35,3 +35,26 @@ def test_every_item_is_taken_once(H, S, dtype):
                                _ref_grads(q, k, v, do, scale)):
         # one key of length 1: dq and dk are exactly zero in the reference
         assert (got.float() - want).norm() <= 1e-2 * want.norm() + 1e-3, name
+
+
+@pytest.mark.parametrize("row_stride", [(1 << 24) - 8, 1 << 24])
+def test_row_strides_around_the_whole_tile_loads(row_stride):
+    """Rows 32 MiB apart: whole tiles go out as one piece below 2^24 elements and load by load
+    from there on; either way the same bits as with dense rows."""
+    S = 70
+    buf = torch.empty(S * row_stride, device="cuda", dtype=torch.bfloat16)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v = dense = [torch.randn(1, 1, S, 128, device="cuda", generator=g).to(torch.bfloat16)
+                       for _ in range(3)]
+    far = [buf.as_strided((1, 1, S, 128), (S * row_stride, 128, row_stride, 1), 128 * i)
+           for i in range(3)]
+    for a, b in zip(far, dense):
+        a.copy_(b)
+    do = torch.randn(1, S, 1, 128, device="cuda", generator=g).to(torch.bfloat16)
+    scale = 1.0 / math.sqrt(128)
+    want = attention.attn_fwd(q, k, v, scale)
+    got = attention.attn_fwd(*far, scale)
+    want += tuple(attention.attn_bwd(q, k, v, *want, do, scale))
+    got += tuple(attention.attn_bwd(*far, *got, do, scale))
+    for name, a, b in zip(("o", "lse", "dq", "dk", "dv"), got, want):
+        assert torch.equal(a, b), name
