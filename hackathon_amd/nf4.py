@@ -270,8 +270,24 @@ def lora_few(x, packed, quant_state, lora_a, lora_b, scaling, bias=None):
     """x @ W^T + bf16(x @ A^T) @ (scaling B)^T (+ bias) for x [M <= 32, K] and an adapter's fp32
     factors A [16, K], B [N, 16], in two launches (qlora_nf4_lora_few)."""
     M, K = x.shape
+    N, K_w = (int(d) for d in quant_state.shape)
+    if K != K_w:
+        raise ValueError(f"x has {K} columns, the weight {K_w}")
+    if lora_a.shape != (16, K) or lora_b.shape != (N, 16):
+        raise ValueError(f"the factors must be [16, {K}] and [{N}, 16], got "
+                         f"{tuple(lora_a.shape)} and {tuple(lora_b.shape)}")
+    if x.dtype not in (torch.bfloat16, torch.float16) or lora_a.dtype != torch.float32 \
+            or lora_b.dtype != torch.float32:
+        raise TypeError(f"x must be bf16 or fp16 and the factors fp32, got {x.dtype}, "
+                        f"{lora_a.dtype}, {lora_b.dtype}")
+    if x.stride(-1) != 1 or not (lora_a.is_contiguous() and lora_b.is_contiguous()
+                                 and packed.is_contiguous()):
+        raise ValueError("x must have unit stride along its rows; the factors and the packed "
+                         "codes must be contiguous")
+    if packed.numel() * packed.element_size() * 2 < N * K:
+        raise ValueError("packed buffer is smaller than the quantised shape")
+    _lib.require_device(x, packed, lora_a, lora_b)
     absmax, nested, code2, absmax2, offset, blocksize2 = _scale_args(quant_state)
-    N = int(quant_state.shape[0])
     out = torch.empty((M, N), dtype=x.dtype, device=x.device)
     ws, ws_bytes = _lib.workspace("qlora_nf4_lora_few_workspace_size", M, K, device=x.device)
     _lib.call("qlora_nf4_lora_few", M, N, K, x.data_ptr(), x.stride(0), packed.data_ptr(),

@@ -1,0 +1,85 @@
+"""The few-row LoRA path (nf4.lora_few, lora.LoraNF4Few) refuses operands its kernels would read
+out of range, before any launch; the launch itself is recorded instead of made."""
+
+import pytest
+import torch
+
+from hackathon_amd import _lib, lora, nf4, quant
+
+K, N = 128, 64
+
+
+@pytest.fixture
+def launches(monkeypatch):
+    calls = []
+    monkeypatch.setattr(_lib, "call", lambda *a: calls.append(a))
+    monkeypatch.setattr(_lib, "stream_of", lambda t: 0)
+    monkeypatch.setattr(_lib, "require_device", lambda *t: None)
+    return calls
+
+
+def _operands():
+    packed, qs = quant.quantize_nf4(torch.randn(N, K), 64)
+    x = torch.randn(2, K).bfloat16()
+    return x, packed, qs, torch.randn(16, K), torch.randn(N, 16)
+
+
+def test_operands_that_fit_are_launched(launches):
+    x, packed, qs, a, b = _operands()
+    assert nf4.lora_few(x, packed, qs, a, b, 2.0).shape == (2, N)
+    assert [c[0] for c in launches] == ["qlora_nf4_lora_few"]
+
+
+@pytest.mark.parametrize("what,error", [
+    ("wide x", ValueError), ("narrow x", ValueError), ("short A", ValueError),
+    ("short B", ValueError), ("rank 8", ValueError), ("fp32 x", TypeError),
+    ("bf16 A", TypeError), ("bf16 B", TypeError), ("strided x", ValueError),
+    ("strided A", ValueError), ("strided B", ValueError), ("few codes", ValueError)])
+def test_operands_that_do_not_fit_raise_before_the_launch(launches, what, error):
+    x, packed, qs, a, b = _operands()
+    if what == "wide x":
+        x = torch.randn(2, 2 * K).bfloat16()
+    elif what == "narrow x":
+        x = x[:, :64].contiguous()
+    elif what == "short A":
+        a = a[:, :64].contiguous()
+    elif what == "short B":
+        b = b[:32]
+    elif what == "rank 8":
+        a, b = a[:8], b[:, :8].contiguous()
+    elif what == "fp32 x":
+        x = x.float()
+    elif what == "bf16 A":
+        a = a.bfloat16()
+    elif what == "bf16 B":
+        b = b.bfloat16()
+    elif what == "strided x":
+        x = torch.randn(2, 2 * K).bfloat16()[:, ::2]
+    elif what == "strided A":
+        a = torch.randn(16, 2 * K)[:, ::2]
+    elif what == "strided B":
+        b = torch.randn(16, N).t()
+    else:
+        packed = packed[: packed.shape[0] // 2]
+    with pytest.raises(error):
+        nf4.lora_few(x, packed, qs, a, b, 2.0)
+    assert not launches
+
+
+def test_operands_off_the_gpu_raise():
+    with pytest.raises(ValueError, match="on a GPU device"):
+        x, packed, qs, a, b = _operands()
+        nf4.lora_few(x, packed, qs, a, b, 2.0)
+
+
+@pytest.mark.parametrize("width", [2 * K, 64])
+def test_layer_of_another_width_raises_without_gradients(launches, width):
+    base = quant.Linear4bit.from_weight(torch.randn(N, K).bfloat16(),
+                                        compute_dtype=torch.bfloat16)
+    layer = lora.LoraLinear4bit(base, compute_dtype=torch.bfloat16)
+    x = torch.randn(2, width).bfloat16()
+    a, b = layer.lora_A["default"].weight, layer.lora_B["default"].weight
+    with torch.no_grad(), pytest.raises(ValueError, match=f"x has {width} columns"):
+        assert lora._takes_few(x, a, b, base.weight, base.weight.quant_state)
+        lora.LoraNF4Few.apply(x, a, b, base.weight, base.weight.quant_state, None, 2.0)
+    assert not launches
