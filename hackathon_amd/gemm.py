@@ -186,6 +186,8 @@ def lora_down(x: torch.Tensor, y: torch.Tensor, out: torch.Tensor, alpha: float 
     _lib.require_rows(x.dtype, x=x, y=y, out_t=out_t)
     _lib.require_rows(out.dtype, out=out)
     M, K = x.shape
+    if y.shape[1] < K:
+        raise ValueError(f"x has {K} columns, the factor {y.shape[1]}")
     slots = _slots(y.shape[0], "y")
     ws, ws_bytes = _lib.workspace("qlora_lora_down_workspace_size", M, K, slots, device=x.device)
     _lib.call("qlora_lora_down", x.data_ptr(), x.stride(0), y.data_ptr(), y.stride(0), M, K,

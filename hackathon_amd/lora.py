@@ -181,6 +181,8 @@ def dropout_down(x2, a16, p, seeds, u, ut=None, keep_xd=False):
     of 64."""
     M, K = x2.shape
     G = len(seeds)
+    if a16.shape[0] < 16 * G or a16.shape[1] < K:
+        raise ValueError(f"x has {K} columns and {G} adapters, A is {tuple(a16.shape)}")
     if x2.data_ptr() % 16 or x2.stride(0) % 8:
         x2 = x2.contiguous() if x2.stride(0) % 8 else x2.clone()
     xds = ([torch.empty((M, K), dtype=x2.dtype, device=x2.device) for _ in range(G)]

@@ -1,5 +1,6 @@
-"""The few-row LoRA path (nf4.lora_few, lora.LoraNF4Few) refuses operands its kernels would read
-out of range, before any launch; the launch itself is recorded instead of made."""
+"""The few-row paths of the 4-bit LoRA layer (nf4.lora_few, lora.LoraNF4Few, LoraNF4Linear up to 256
+rows) refuse operands their kernels would read out of range, before any launch; the launches are
+recorded instead of made."""
 
 import pytest
 import torch
@@ -82,4 +83,19 @@ def test_layer_of_another_width_raises_without_gradients(launches, width):
     with torch.no_grad(), pytest.raises(ValueError, match=f"x has {width} columns"):
         assert lora._takes_few(x, a, b, base.weight, base.weight.quant_state)
         lora.LoraNF4Few.apply(x, a, b, base.weight, base.weight.quant_state, None, 2.0)
+    assert not launches
+
+
+@pytest.mark.parametrize("p", [0.0, 0.1])
+def test_layer_of_another_width_raises_with_gradients(launches, monkeypatch, p):
+    """The path with gradients forms the down-projection before its GEMM compares the widths: a
+    wider x must not get as far as reading past A."""
+    packed, qs = quant.quantize_nf4(torch.randn(N, K), 64)
+    a, b = torch.randn(16, K).requires_grad_(), torch.randn(N, 16).requires_grad_()
+    t = torch.zeros(16, K, dtype=torch.bfloat16)
+    monkeypatch.setattr(lora.adapter_packs, "pack", lambda *_: (t, t, t, t))
+    monkeypatch.setattr(_lib, "require_rows", lambda dtype, **_: None)
+    x = torch.randn(2, 2 * K).bfloat16()
+    with pytest.raises(ValueError, match=f"x has {2 * K} columns"):
+        lora.LoraNF4Linear.apply(x, a, b, packed, qs, None, 2.0, p, 1)
     assert not launches
