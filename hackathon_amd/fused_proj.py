@@ -364,7 +364,7 @@ class LoraMLP(torch.autograd.Function):
                                               seeds[:2] if specs[0].p > 0 else None)
         n, N = specs[0].n, dspec.n
         a16_d, at_d, bs_d, bt_d = adapter_packs.pack(ab[4], ab[5], dspec.scaling, dt, _PAD)
-        bias = None if dspec.bias is None else dspec.bias.to(dt)
+        bias = None if dspec.bias is None else dspec.bias.to(dt).contiguous()
         res2 = None if residual is None else residual.view(M, N)
         if M > nf4.FUSED_GEMM_MAX_ROWS or not nf4.fused_gemm_ok(dspec.qs, dspec.packed):
             (weight,), table, stream = _native_args((dspec,), y)

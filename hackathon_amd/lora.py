@@ -255,7 +255,7 @@ class LoraNF4Linear(torch.autograd.Function):
         N = int(quant_state.shape[0])
         # A, A^T|0, s*B|0 and B^T in the compute dtype, one launch (kept for the backward)
         a16, at, bs, bt = adapter_packs.pack(a_weight, b_weight, scaling, dt, _PAD)
-        b16 = None if bias is None else bias.to(dt)
+        b16 = None if bias is None else bias.to(dt).contiguous()
         bits = None
         if M > nf4.FUSED_GEMM_MAX_ROWS or not nf4.fused_gemm_ok(quant_state, packed, x2):
             y, ut, bitss = _host.load().group_forward(
@@ -314,8 +314,7 @@ class LoraNF4Few(torch.autograd.Function):
         from . import nf4
 
         x2 = x.reshape(-1, x.shape[-1])
-        y = nf4.lora_few(x2, packed, quant_state, a_weight, b_weight, scaling,
-                         None if bias is None else bias.to(x.dtype))
+        y = nf4.lora_few(x2, packed, quant_state, a_weight, b_weight, scaling, bias)
         return y.view(*x.shape[:-1], y.shape[-1])
 
 

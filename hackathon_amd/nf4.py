@@ -286,7 +286,11 @@ def lora_few(x, packed, quant_state, lora_a, lora_b, scaling, bias=None):
                          "codes must be contiguous")
     if packed.numel() * packed.element_size() * 2 < N * K:
         raise ValueError("packed buffer is smaller than the quantised shape")
-    _lib.require_device(x, packed, lora_a, lora_b)
+    if bias is not None:
+        if bias.numel() != N:
+            raise ValueError(f"bias has {bias.numel()} elements, the output {N} columns")
+        bias = bias.to(x.dtype).contiguous()
+    _lib.require_device(x, packed, lora_a, lora_b, bias)
     absmax, nested, code2, absmax2, offset, blocksize2 = _scale_args(quant_state)
     out = torch.empty((M, N), dtype=x.dtype, device=x.device)
     ws, ws_bytes = _lib.workspace("qlora_nf4_lora_few_workspace_size", M, K, device=x.device)

@@ -2,6 +2,8 @@
 rows) refuse operands their kernels would read out of range, before any launch; the launches are
 recorded instead of made."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -99,3 +101,39 @@ def test_layer_of_another_width_raises_with_gradients(launches, monkeypatch, p):
     with pytest.raises(ValueError, match=f"x has {2 * K} columns"):
         lora.LoraNF4Linear.apply(x, a, b, packed, qs, None, 2.0, p, 1)
     assert not launches
+
+
+def _dense_at(address, n):
+    return torch.frombuffer((ctypes.c_char * (2 * n)).from_address(address),
+                            dtype=torch.bfloat16).clone()
+
+
+def test_strided_bias_reaches_the_few_row_launch_dense(launches, monkeypatch):
+    x, packed, qs, a, b = _operands()
+    bias = torch.randn(N, 2).bfloat16()[:, 0]
+    seen = []
+    monkeypatch.setattr(_lib, "call", lambda *args: seen.append(_dense_at(args[-4], N)))
+    lora.LoraNF4Few.apply(x, a, b, packed, qs, bias, 2.0)
+    assert torch.equal(seen[0], bias)
+    with pytest.raises(ValueError, match="bias"):
+        lora.LoraNF4Few.apply(x, a, b, packed, qs, bias[:32], 2.0)
+
+
+def test_strided_bias_reaches_the_native_calls_dense(launches, monkeypatch):
+    packed, qs = quant.quantize_nf4(torch.randn(N, K), 64)
+    a, b = torch.randn(16, K), torch.randn(N, 16)
+    t = torch.zeros(16, K, dtype=torch.bfloat16)
+    monkeypatch.setattr(lora.adapter_packs, "pack", lambda *_: (t, t, t, t))
+    seen = []
+
+    class Host:
+        @staticmethod
+        def group_forward(x, a16, bs, weights, bias, *rest):
+            seen.append(bias)
+            return torch.zeros(x.shape[0], N), t, []
+
+    monkeypatch.setattr(lora._host, "load", lambda: Host)
+    bias = torch.randn(N, 2).bfloat16()[:, 0]
+    lora.LoraNF4Linear.apply(torch.randn(300, K).bfloat16(), a, b, packed, qs, bias, 2.0,
+                             0.0, 0)
+    assert seen[0].is_contiguous() and torch.equal(seen[0], bias)

@@ -1,0 +1,44 @@
+"""The 4-bit LoRA layers whose launches the native host code queues (csrc/host/host.cpp), at the
+operand forms a caller may hand in, against an fp64 product."""
+
+import pytest
+import torch
+
+from hackathon_amd import lora, nf4, quant
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(N, K, seed, dtype=torch.bfloat16):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    packed, st = quant.quantize_nf4(torch.randn(N, K, device="cuda", generator=g) * 0.02, 64)
+    a = torch.randn(16, K, device="cuda", generator=g) / K ** 0.5
+    b = torch.randn(N, 16, device="cuda", generator=g) * 0.05
+    return g, packed, st, a, b
+
+
+def _check(y, x, packed, st, a, b, bias, dtype=torch.bfloat16):
+    w = nf4.dequantize_nf4(packed, st, dtype).double()
+    K = w.shape[1]
+    a16, sb = a.to(dtype).double(), (2.0 * b).to(dtype).double()
+    u = x.double() @ a16.t()
+    ref = x.double() @ w.t() + u @ sb.t() + bias.double()
+    mag = x.double().abs() @ w.abs().t() + (x.double().abs() @ a16.abs().t()) @ sb.abs().t()
+    # fp32 accumulation over K + 16 terms, u rounded once, then one rounding to the output
+    ulp16 = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    bound = ((K + 32) * 2.0 ** -24 * mag + ulp16 * (u.abs() @ sb.abs().t()) + ulp16 * ref.abs()
+             + 1e-6)
+    assert torch.all((y.double() - ref).abs() <= bound)
+
+
+@pytest.mark.parametrize("M", [3, 40, 300])
+def test_strided_bias(M):
+    """A bias that is a column of a wider tensor, already in the compute dtype."""
+    print(f"strided bias M={M}", flush=True)
+    g, packed, st, a, b = _layer(256, 128, M)
+    x = torch.randn(M, 128, device="cuda", generator=g).bfloat16()
+    bias = torch.randn(256, 3, device="cuda", generator=g).bfloat16()[:, 1]
+    if M <= nf4.LORA_FEW_MAX_ROWS:
+        _check(lora.LoraNF4Few.apply(x, a, b, packed, st, bias, 2.0), x, packed, st, a, b, bias)
+    y = lora.LoraNF4Linear.apply(x, a, b, packed, st, bias, 2.0, 0.0, 0)
+    _check(y, x, packed, st, a, b, bias)
