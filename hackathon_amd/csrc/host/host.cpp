@@ -144,7 +144,7 @@ struct Weight {
   int64_t n, k;
 
   ql_nf4_weight desc(void* out) const {
-    return {packed.data_ptr<uint8_t>(), n, k, absmax.data_ptr(),
+    return {static_cast<const uint8_t*>(packed.data_ptr()), n, k, absmax.data_ptr(),
             static_cast<const float*>(ptr(code2)), static_cast<const float*>(ptr(absmax2)),
             offset, bs, bs2, out};
   }
@@ -163,7 +163,8 @@ Weight weight(const py::handle& h) {
   w.n = t[8].cast<int64_t>();
   w.k = t[9].cast<int64_t>();
   TORCH_CHECK_VALUE(w.packed.is_cuda(), "HIP kernels need tensors on a GPU device");
-  TORCH_CHECK_VALUE(w.packed.is_contiguous() && w.packed.numel() * 2 >= w.n * w.k,
+  // two weights a byte, whatever type the bytes are stored as
+  TORCH_CHECK_VALUE(w.packed.is_contiguous() && (int64_t)w.packed.nbytes() * 2 >= w.n * w.k,
                     "packed buffer is smaller than the quantised shape");
   return w;
 }
@@ -181,6 +182,8 @@ void dequant(const Ctx& c, const std::vector<Weight>& ws, const Tensor& w) {
   int64_t off = 0;
   std::vector<char*> outs;
   for (const auto& x : ws) {
+    TORCH_CHECK_VALUE(x.packed.numel() * 2 >= x.n * x.k,
+                      "packed buffer is smaller than the quantised shape");
     char* out = static_cast<char*>(w.data_ptr()) + 2 * off * x.k;
     outs.push_back(out);
     off += x.n;

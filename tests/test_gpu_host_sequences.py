@@ -42,3 +42,31 @@ def test_strided_bias(M):
         _check(lora.LoraNF4Few.apply(x, a, b, packed, st, bias, 2.0), x, packed, st, a, b, bias)
     y = lora.LoraNF4Linear.apply(x, a, b, packed, st, bias, 2.0, 0.0, 0)
     _check(y, x, packed, st, a, b, bias)
+
+
+def _step(x, packed, st, a, b, dy):
+    a, b, x = (t.detach().clone().requires_grad_() for t in (a, b, x))
+    y = lora.LoraNF4Linear.apply(x, a, b, packed, st, None, 2.0, 0.0, 0)
+    return [y.detach(), *torch.autograd.grad(y, [x, a, b], dy)]
+
+
+@pytest.mark.parametrize("M,storage", [(300, torch.int8), (40, torch.int8), (40, torch.bfloat16)])
+def test_codes_stored_as_another_type(M, storage):
+    """The packed bytes held by a tensor of another type (bitsandbytes' quant_storage): the same
+    bits as from uint8, forward and backward. A type wider than a byte is taken up to 256 rows;
+    above, the forward refuses a buffer with fewer than half as many elements as weights."""
+    print(f"codes stored as {storage} M={M}", flush=True)
+    g, packed, st, a, b = _layer(256, 128, M)
+    x = torch.randn(M, 128, device="cuda", generator=g).bfloat16()
+    dy = torch.randn(M, 256, device="cuda", generator=g).bfloat16()
+    want = _step(x, packed, st, a, b, dy)
+    got = _step(x, packed.view(-1).view(storage), st, a, b, dy)
+    assert all(torch.equal(p, q) for p, q in zip(got, want))
+
+
+def test_wide_codes_refused_by_the_dense_forward():
+    g, packed, st, a, b = _layer(256, 128, 1)
+    x = torch.randn(300, 128, device="cuda", generator=g).bfloat16()
+    with pytest.raises(ValueError, match="packed buffer is smaller"):
+        lora.LoraNF4Linear.apply(x, a, b, packed.view(-1).view(torch.bfloat16), st, None, 2.0,
+                                 0.0, 0)
