@@ -511,6 +511,13 @@ py::tuple py_mlp_down(const Tensor& y, const Tensor& a16, const Tensor& bs, cons
     const int64_t M = y.size(0), n = wd[0].k, N = wd[0].n;
     TORCH_CHECK_VALUE(y.size(1) == 2 * n && a16.size(1) == n && bs.size(0) == N,
                       "the down projection does not fit gate and up");
+    if (residual_.has_value() && !bias_.has_value()) {  // the GEMM adds it: read as y's type
+      const Tensor& t = *residual_;
+      TORCH_CHECK_VALUE(t.is_cuda() && t.scalar_type() == y.scalar_type(),
+                        "a residual takes no bias, alpha 1 and out's dtype");
+      TORCH_CHECK_VALUE(t.dim() == 2 && t.size(0) == M && t.size(1) == N && t.stride(1) == 1,
+                        "residual must be [", M, ", ", N, "] with unit column stride");
+    }
     const Tensor h = c.empty(M, n), u = c.empty(M, kPad);
     ut = c.t_buffer(16, M);
     const Mat gate = cols16(y, 0, n), up = cols16(y, n, 2 * n);
@@ -534,7 +541,7 @@ py::tuple py_mlp_down(const Tensor& y, const Tensor& a16, const Tensor& bs, cons
     const Tensor w = c.empty(N, n), bias = bias_.value_or(Tensor());
     const Tensor res = residual_.value_or(Tensor());
     dequant(c, wd, w);
-    const bool fused = res.defined() && !bias.defined();
+    const bool fused = res.defined() && !bias.defined();  // else torch adds it
     gemm(c, mat(h), mat(w), mat(u), mat(bs), mat(out), bias, fused ? res : Tensor());
     if (res.defined() && !fused) out = res + out;
   }

@@ -42,3 +42,52 @@ def test_weight_args_hold_a_contiguous_copy_of_strided_codes():
     args = nf4.weight_args(wide[:, :1], qs)
     assert args[0].is_contiguous() and torch.equal(args[0], packed)
     assert args[-2:] == (64, 128)
+
+
+# ---- refusals that come after the device check: tensors with a GPU's device and no storage ----
+M, K, N, PAD = 300, 128, 64, 64
+
+
+@pytest.fixture
+def fake():
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    host = _host.load()  # outside the mode
+    with FakeTensorMode():
+        yield host
+
+
+def _t(*shape, dtype=torch.bfloat16):
+    return torch.empty(*shape, dtype=dtype, device="cuda:0")
+
+
+def _w(n, k):
+    return (_t(n * k // 2, dtype=torch.uint8), _t(n * k // 64, dtype=torch.uint8), 1,
+            _t(256, dtype=torch.float32), _t(n * k // 64, dtype=torch.float32), 0.0, 64, 256, n, k)
+
+
+TABLE = torch.zeros(16)
+
+
+def _refused(error, match, call, args, **changes):
+    """call() with some operands replaced raises before any launch; as they are, they get as far as
+    the first launch, which refuses their null pointers."""
+    with pytest.raises(error, match=match):
+        call(*{**args, **changes}.values())
+    with pytest.raises(RuntimeError, match="null pointer|not allocated"):
+        call(*args.values())
+
+
+def _down_args():
+    return dict(y=_t(M, 2 * K), a16=_t(16, K), bs=_t(N, PAD), spec=_w(N, K), bias=None,
+                residual=_t(M, N), p=0.0, seed=0, table=TABLE, stream=0)
+
+
+@pytest.mark.parametrize("residual,match", [
+    (lambda: _t(M, N, dtype=torch.float32), "out's dtype"),
+    (lambda: _t(M, N // 2), "residual must be"),
+    (lambda: _t(M - 1, N), "residual must be"),
+    (lambda: _t(M, 2 * N)[:, ::2], "residual must be"),
+    (lambda: torch.empty(M, N, dtype=torch.bfloat16), "out's dtype")])
+def test_mlp_down_refuses_a_residual_the_gemm_would_misread(fake, residual, match):
+    _refused(ValueError, match, fake.mlp_down, _down_args(), residual=residual())
