@@ -574,9 +574,12 @@ py::tuple py_mlp_backward(const Tensor& dy, const Tensor& x, const Tensor& y, co
     TORCH_CHECK_VALUE(dy.size(0) == M && dy.size(1) == N && y.size(1) == 2 * n && ws.size() == 2 &&
                           scaling.size() == 2 && need.size() == 6 && bt.size(1) == 2 * n,
                       "the MLP's operands do not fit together");
-    TORCH_CHECK_VALUE(ut.stride(0) == ut_d.stride(0), "ut and ut_d must share a row stride");
     Tensor du_d = c.empty(M, kPad);
     const Tensor dut_d = c.t_buffer(16, M);
+    // the SwiGLU kernel takes one row stride for all three (a saved-tensor hook may have packed
+    // the forward's anew)
+    TORCH_CHECK_VALUE(ut.stride(0) == dut_d.stride(0) && ut_d.stride(0) == dut_d.stride(0),
+                      "ut, ut_d and du_d^T must share a row stride");
     lora_down(c, mat(dy), mat(bt_d), (float)s_d, mat(du_d), mat(dut_d));
     const bool masked = bits_d.has_value();
     Tensor dh = c.empty(M, n);

@@ -91,3 +91,25 @@ def _down_args():
     (lambda: torch.empty(M, N, dtype=torch.bfloat16), "out's dtype")])
 def test_mlp_down_refuses_a_residual_the_gemm_would_misread(fake, residual, match):
     _refused(ValueError, match, fake.mlp_down, _down_args(), residual=residual())
+
+
+def _t_t(rows, m=M, ld=304):
+    return _t(rows, ld)[:, :m]
+
+
+def _mlp_args():
+    return dict(dy=_t(M, N), x=_t(M, K), y=_t(M, 2 * K), at=_t(K, PAD), bt=_t(32, 2 * K),
+                ut=_t_t(32), specs=[_w(K, K), _w(K, K)], scaling=[2.0, 2.0], p=0.0, a16=None,
+                bits=[], at_d=_t(K, PAD), bt_d=_t(16, N), ut_d=_t_t(16), spec_d=_w(N, K), s_d=2.0,
+                p_d=0.0, a16_d=None, bits_d=None, need_dx=True, need=[True] * 6, table=TABLE,
+                stream=0)
+
+
+@pytest.mark.parametrize("change", [dict(ut=300, ut_d=300), dict(ut=312, ut_d=312), dict(ut=312),
+                                    dict(ut_d=312)])
+def test_mlp_backward_refuses_transposed_operands_of_another_row_stride(fake, change):
+    """The SwiGLU kernel reads ut, ut_d and the du_d^T made here by one row stride (304 for 300
+    rows); saved-tensor hooks may hand the first two back packed otherwise."""
+    rows = {"ut": 32, "ut_d": 16}
+    _refused(ValueError, "row stride", fake.mlp_backward, _mlp_args(),
+             **{n: _t_t(rows[n], ld=ld) for n, ld in change.items()})
