@@ -87,6 +87,22 @@ void rows(const Tensor& t, at::ScalarType dtype, const char* name) {
                     " must be a 2-D matrix with unit stride along its rows");
 }
 
+// Such a matrix of at least r x c, what the kernels read of it.
+void matrix(const Tensor& t, at::ScalarType dtype, int64_t r, int64_t c, const char* name) {
+  rows(t, dtype, name);
+  TORCH_CHECK_VALUE(t.size(0) >= r && t.size(1) >= c, name, " is [", t.size(0), ", ", t.size(1),
+                    "]; this call reads [", r, ", ", c, "]");
+}
+
+// A GEMM's bias: n consecutive values.
+void vec(const Tensor& t, at::ScalarType dtype, int64_t n, const char* name) {
+  TORCH_CHECK_VALUE(t.is_cuda(), name, " must be on a GPU device");
+  TORCH_CHECK_TYPE(t.scalar_type() == dtype, name, " is ", t.scalar_type(), "; this call takes ",
+                   dtype, " operands");
+  TORCH_CHECK_VALUE(t.numel() == n && t.is_contiguous(), name, " must be ", n,
+                    " consecutive values");
+}
+
 bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 bool pow2(int64_t v) { return v > 0 && (v & (v - 1)) == 0; }
 
@@ -266,6 +282,11 @@ Tensor lora_wgrad(const Ctx& c, Mat pt, Mat q, float alpha, bool transposed) {
   return out;
 }
 
+// The keep bits of G adapters' inputs [M, K].
+void keep_bits(const std::vector<Tensor>& bits, int64_t G, int64_t M, int64_t K) {
+  TORCH_CHECK_VALUE((int64_t)bits.size() == G, "one keep-bit tensor per adapter");
+  for (const auto& b : bits) matrix(b, at::kByte, (M + 7) / 8, K, "bits");
+}
 std::vector<const uint8_t*> bit_ptrs(const std::vector<Tensor>& bits) {
   std::vector<const uint8_t*> p;
   for (const auto& b : bits) {
@@ -301,6 +322,7 @@ GroupForward group_forward(const Ctx& c, const Tensor& x, const Tensor& a16, con
   }
   TORCH_CHECK_VALUE(a16.size(0) == 16 * G && a16.size(1) == K && bs.size(0) == N &&
                         bs.size(1) == kPad, "the packed adapters do not fit the group");
+  if (bias.defined()) vec(bias, x.scalar_type(), N, "bias");
   GroupForward r;
   const Tensor u = c.empty(M, kPad);
   r.ut = c.t_buffer(16 * G, M);
@@ -328,7 +350,7 @@ GroupForward group_forward(const Ctx& c, const Tensor& x, const Tensor& a16, con
   // a wide projection gets its own GEMM, narrow neighbours share one
   int64_t c0 = 0, width = 0;
   auto emit = [&](int64_t c1) {
-    Tensor b = bias.defined() ? bias.narrow(0, c0, c1 - c0) : Tensor();
+    Tensor b = bias.defined() ? bias.view(-1).narrow(0, c0, c1 - c0) : Tensor();
     gemm(c, mat(x), rows16(w, c0, c1), mat(u), rows16(bs, c0, c1), cols16(r.y, c0, c1), b,
          Tensor());
     c0 = c1;
@@ -364,6 +386,21 @@ GroupBackward group_backward(const Ctx& c, const Tensor& g, const Tensor& x, con
   TORCH_CHECK_VALUE(g.size(1) == N && x.size(0) == M && at_pad.size(0) == K && bt.size(1) == N &&
                         (int64_t)scaling.size() == G && (int64_t)need.size() == 2 * G,
                     "the group's operands do not fit together");
+  const auto dt = x.scalar_type();
+  matrix(bt, dt, 16 * G, N, "bt");
+  matrix(ut, dt, 16 * G, M, "ut");
+  TORCH_CHECK_VALUE(du.defined() == dut.defined(), "du and its transpose come together");
+  if (du.defined()) {
+    matrix(du, dt, M, 16 * G, "du");
+    matrix(dut, dt, 16 * G, M, "dut");
+  }
+  matrix(at_pad, dt, K, du.defined() ? du.size(1) : kPad, "at");
+  TORCH_CHECK_VALUE(db_given.empty() || (int64_t)db_given.size() == G,
+                    "one lora_B gradient per adapter");
+  if (drop.p > 0) {
+    matrix(drop.a16, dt, 16 * G, K, "a16");
+    keep_bits(drop.bits, G, M, K);
+  }
   bool same = true;
   for (const double s : scaling) same = same && s == scaling[0];
   if (!du.defined()) {
@@ -511,6 +548,9 @@ py::tuple py_mlp_down(const Tensor& y, const Tensor& a16, const Tensor& bs, cons
     const int64_t M = y.size(0), n = wd[0].k, N = wd[0].n;
     TORCH_CHECK_VALUE(y.size(1) == 2 * n && a16.size(1) == n && bs.size(0) == N,
                       "the down projection does not fit gate and up");
+    matrix(a16, y.scalar_type(), 16, n, "a16");
+    matrix(bs, y.scalar_type(), N, kPad, "bs");
+    if (bias_.has_value()) vec(*bias_, y.scalar_type(), N, "bias");
     if (residual_.has_value() && !bias_.has_value()) {  // the GEMM adds it: read as y's type
       const Tensor& t = *residual_;
       TORCH_CHECK_VALUE(t.is_cuda() && t.scalar_type() == y.scalar_type(),
@@ -574,6 +614,19 @@ py::tuple py_mlp_backward(const Tensor& dy, const Tensor& x, const Tensor& y, co
     TORCH_CHECK_VALUE(dy.size(0) == M && dy.size(1) == N && y.size(1) == 2 * n && ws.size() == 2 &&
                           scaling.size() == 2 && need.size() == 6 && bt.size(1) == 2 * n,
                       "the MLP's operands do not fit together");
+    const bool masked = bits_d.has_value();
+    matrix(y, dt, M, 2 * n, "y");
+    matrix(bt, dt, 32, 2 * n, "bt");
+    matrix(ut, dt, 32, M, "ut");
+    matrix(bt_d, dt, 16, N, "bt_d");
+    matrix(ut_d, dt, 16, M, "ut_d");
+    if (masked) {
+      TORCH_CHECK_VALUE(a16_d.has_value(), "dropout needs the down adapter's A");
+      matrix(*a16_d, dt, 16, n, "a16_d");
+      keep_bits({*bits_d}, 1, M, n);
+    } else {
+      matrix(at_d, dt, n, kPad, "at_d");
+    }
     Tensor du_d = c.empty(M, kPad);
     const Tensor dut_d = c.t_buffer(16, M);
     // the SwiGLU kernel takes one row stride for all three (a saved-tensor hook may have packed
@@ -581,7 +634,6 @@ py::tuple py_mlp_backward(const Tensor& dy, const Tensor& x, const Tensor& y, co
     TORCH_CHECK_VALUE(ut.stride(0) == dut_d.stride(0) && ut_d.stride(0) == dut_d.stride(0),
                       "ut, ut_d and du_d^T must share a row stride");
     lora_down(c, mat(dy), mat(bt_d), (float)s_d, mat(du_d), mat(dut_d));
-    const bool masked = bits_d.has_value();
     Tensor dh = c.empty(M, n);
     {
       const Tensor wt = c.empty(n, N);
@@ -611,7 +663,6 @@ py::tuple py_mlp_backward(const Tensor& dy, const Tensor& x, const Tensor& y, co
                 dut.stride(0), db_g.data_ptr<float>(), db_u.data_ptr<float>(), dut_d.data_ptr(),
                 1.0f, da_d.data_ptr<float>(), ptr(wk), bytes, c.stream);
       } else {
-        TORCH_CHECK_VALUE(a16_d.has_value(), "dropout needs the down adapter's A");
         QL_CALL(qlora_swiglu_bwd_lora_dropout, dh.data_ptr(), dh.stride(0), gate.p, gate.ld, up.p,
                 up.ld, dg.p, dg.ld, dup.p, dup.ld, M, n, bt_g.p, bt_u.p, bt_g.ld, ut_g.p, ut_u.p,
                 ut_g.ld, sg, su, sg, su, c.dt, du.data_ptr(), du.stride(0), (int)kPad,

@@ -113,3 +113,73 @@ def test_mlp_backward_refuses_transposed_operands_of_another_row_stride(fake, ch
     rows = {"ut": 32, "ut_d": 16}
     _refused(ValueError, "row stride", fake.mlp_backward, _mlp_args(),
              **{n: _t_t(rows[n], ld=ld) for n, ld in change.items()})
+
+
+def _f32(*shape):
+    return _t(*shape, dtype=torch.float32)
+
+
+def _bits(m=M, k=K):
+    return _t((m + 7) // 8, k, dtype=torch.uint8)
+
+
+@pytest.mark.parametrize("error,match,change", [
+    (TypeError, "bt is Float", lambda: dict(bt=_f32(32, 2 * K))),
+    (ValueError, "bt is .16", lambda: dict(bt=_t(16, 2 * K))),
+    (ValueError, "ut is .16", lambda: dict(ut=_t_t(16))),
+    (TypeError, "at_d is Float", lambda: dict(at_d=_f32(K, PAD))),
+    (ValueError, "at_d is", lambda: dict(at_d=_t(K, 16))),
+    (TypeError, "bt_d is Float", lambda: dict(bt_d=_f32(16, N))),
+    (ValueError, "bt_d is", lambda: dict(bt_d=_t(16, N // 2))),
+    (ValueError, "ut_d is", lambda: dict(ut_d=_t_t(16, M - 8))),
+    (ValueError, "y is", lambda: dict(y=_t(M - 1, 2 * K))),
+    (TypeError, "bits is", lambda: dict(bits_d=_t(38, K), a16_d=_t(16, K), p_d=0.1)),
+    (ValueError, "bits is", lambda: dict(bits_d=_bits(M - 8), a16_d=_t(16, K), p_d=0.1)),
+    (TypeError, "a16_d is Float", lambda: dict(bits_d=_bits(), a16_d=_f32(16, K), p_d=0.1)),
+    (ValueError, "needs the down adapter's A", lambda: dict(bits_d=_bits(), p_d=0.1))])
+def test_mlp_backward_refuses_operands_the_kernels_would_misread(fake, error, match, change):
+    _refused(error, match, fake.mlp_backward, _mlp_args(), **change())
+
+
+def _group_args():
+    return dict(g=_t(M, 2 * N), x=_t(M, K), at=_t(K, PAD), bt=_t(32, 2 * N), ut=_t_t(32),
+                specs=[_w(N, K), _w(N, K)], scaling=[2.0, 2.0], need_dx=True, need=[True] * 4,
+                du=None, dut=None, db=[], p=0.0, a16=None, bits=[], table=TABLE, stream=0)
+
+
+@pytest.mark.parametrize("error,match,change", [
+    (ValueError, "bt is .16", lambda: dict(bt=_t(16, 2 * N))),
+    (ValueError, "ut is .16", lambda: dict(ut=_t_t(16))),
+    (ValueError, "ut is", lambda: dict(ut=_t_t(32, M - 8))),
+    (ValueError, "at is", lambda: dict(at=_t(K, 32))),
+    (ValueError, "come together", lambda: dict(du=_t(M, PAD))),
+    (TypeError, "du is Float", lambda: dict(du=_f32(M, PAD), dut=_t_t(32))),
+    (ValueError, "du is", lambda: dict(du=_t(M - 1, PAD), dut=_t_t(32))),
+    (ValueError, "dut is", lambda: dict(du=_t(M, PAD), dut=_t_t(16))),
+    (ValueError, "one lora_B gradient", lambda: dict(db=[_f32(N, 16)])),
+    (ValueError, "one keep-bit", lambda: dict(p=0.1, a16=_t(32, K), bits=[_bits()])),
+    (ValueError, "bits is", lambda: dict(p=0.1, a16=_t(32, K), bits=[_bits(), _bits(M - 8)])),
+    (TypeError, "a16 is Float", lambda: dict(p=0.1, a16=_f32(32, K), bits=[_bits(), _bits()])),
+    (ValueError, "a16 is", lambda: dict(p=0.1, a16=_t(16, K), bits=[_bits(), _bits()]))])
+def test_group_backward_refuses_operands_the_kernels_would_misread(fake, error, match, change):
+    _refused(error, match, fake.group_backward, _group_args(), **change())
+
+
+@pytest.mark.parametrize("error,match,bias", [
+    (TypeError, "bias is Float", lambda: _f32(2 * N)),
+    (ValueError, "bias must be 128", lambda: _t(N)),
+    (ValueError, "bias must be 128", lambda: _t(4 * N)[::2]),
+    (ValueError, "bias must be on", lambda: torch.empty(2 * N, dtype=torch.bfloat16))])
+def test_group_forward_and_mlp_down_refuse_a_bias_the_gemm_would_misread(fake, error, match, bias):
+    args = dict(x=_t(M, K), a16=_t(32, K), bs=_t(2 * N, PAD), specs=[_w(N, K), _w(N, K)],
+                bias=None, p=0.0, seeds=[], table=TABLE, stream=0)
+    _refused(error, match, fake.group_forward, args, bias=bias())
+    down = {**_down_args(), "residual": None, "bs": _t(2 * N, PAD), "spec": _w(2 * N, K)}
+    _refused(error, match, fake.mlp_down, down, bias=bias())
+
+
+@pytest.mark.parametrize("error,match,change", [
+    (ValueError, "a16 is", lambda: dict(a16=_t(8, K))),
+    (ValueError, "bs is", lambda: dict(bs=_t(N, 16)))])
+def test_mlp_down_refuses_short_adapters(fake, error, match, change):
+    _refused(error, match, fake.mlp_down, _down_args(), **change())
