@@ -38,6 +38,12 @@ def load():
             spec = importlib.util.spec_from_file_location(name, MODULE_PATH, loader=loader)
             module = importlib.util.module_from_spec(spec)
             loader.exec_module(module)
+            version = getattr(module, "abi_version", None)
+            if version != _lib.ABI_VERSION:
+                raise _lib.KernelLibraryMissing(
+                    f"{MODULE_PATH.name} was built for C-ABI version {version}, the kernel "
+                    f"library has {_lib.ABI_VERSION}: rebuild both with "
+                    f"`python -m hackathon_amd.build`")
             _module = module
         _module.bind([ctypes.cast(getattr(lib, n), ctypes.c_void_p).value
                       for n in _module.entry_names()])

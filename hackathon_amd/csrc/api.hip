@@ -1,7 +1,7 @@
 // Library identification and status text for the C-ABI.
 #include "ql_common.h"
 
-extern "C" int qlora_abi_version(void) { return 3; }
+extern "C" int qlora_abi_version(void) { return QLORA_ABI_VERSION; }
 
 extern "C" const char* qlora_strerror(int status) {
   switch (status) {

@@ -688,6 +688,8 @@ py::tuple py_mlp_backward(const Tensor& dy, const Tensor& x, const Tensor& y, co
 }  // namespace
 
 PYBIND11_MODULE(_qlora_host, m) {
+  // of the signatures it calls by address: compared with the kernel library's before binding
+  m.attr("abi_version") = QLORA_ABI_VERSION;
   m.def("entry_names", &entry_names);
   m.def("bind", &bind);
   m.def("group_forward", &py_group_forward);

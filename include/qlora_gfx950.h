@@ -37,9 +37,10 @@ enum {
 
 typedef void* ql_stream_t; /* hipStream_t */
 
-/* Library identification and error text. qlora_abi_version() is 3 for the signatures in this
- * file (version 1 had no `slots` argument in the qlora_lora_down / qlora_lora_wgrad family;
+/* Library identification and error text. qlora_abi_version() is QLORA_ABI_VERSION for the
+ * signatures in this file (version 1 had no `slots` argument in the qlora_lora_down / qlora_lora_wgrad family;
  * version 2 wrote qlora_lora_pack_group's bt as [16, N] instead of [16 count, N]). */
+#define QLORA_ABI_VERSION 3
 int qlora_abi_version(void);
 const char* qlora_strerror(int status);
 

@@ -183,3 +183,22 @@ def test_group_forward_and_mlp_down_refuse_a_bias_the_gemm_would_misread(fake, e
     (ValueError, "bs is", lambda: dict(bs=_t(N, 16)))])
 def test_mlp_down_refuses_short_adapters(fake, error, match, change):
     _refused(error, match, fake.mlp_down, _down_args(), **change())
+
+
+def test_module_of_another_abi_version_is_refused(monkeypatch):
+    """The module calls the kernel library by address with the signatures it was built from."""
+    assert _host.load().abi_version == _lib.ABI_VERSION == _lib.load().qlora_abi_version()
+    monkeypatch.setattr(_host, "_module", None)
+    monkeypatch.setattr(_host, "_bound", None)
+    real = _host.importlib.machinery.ExtensionFileLoader.exec_module
+    bound = []
+
+    def stale(loader, module):
+        real(loader, module)
+        module.abi_version = _lib.ABI_VERSION - 1
+        module.bind = bound.append
+
+    monkeypatch.setattr(_host.importlib.machinery.ExtensionFileLoader, "exec_module", stale)
+    with pytest.raises(_lib.KernelLibraryMissing, match="C-ABI version"):
+        _host.load()
+    assert not bound and _host._module is None
