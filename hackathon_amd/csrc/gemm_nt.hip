@@ -1163,10 +1163,9 @@ int ql_gemm_nt_auto_splits(int64_t M, int64_t N, int64_t K, bool accumulate) {
   return accumulate ? auto_splits_bn(M, N, K, 32 * choose_nb(M, N)) : plan_nt(M, N, K).splits;
 }
 
-// The same count as the dense product of these sizes, so that both are the same sum (beyond
-// kNf4Rows rows only callers that ask for it take the packed operand).
-int ql_gemm_nf4_auto_splits(int64_t M, int64_t N, int64_t K) {
-  return M <= kNf4Rows ? auto_splits_bn(M, N, K, 256) : plan_nt(M, N, K).splits;
+// The packed operand's only tile is 256 x 256, and this its split count.
+static int ql_gemm_nf4_auto_splits(int64_t M, int64_t N, int64_t K) {
+  return auto_splits_bn(M, N, K, 256);
 }
 
 int ql_gemm_nt2(int in_dtype, int c_dtype, int64_t M, int64_t N, int64_t K, const void* A,
@@ -1253,10 +1252,27 @@ int log2_exact(int64_t v) {  // log2 of a power of two, else -1
   return l;
 }
 
+// The product is the dense one's sum, bit for bit, so it needs the dense plan's split count.
+// Where that is not the count the packed tile wants (the plan went to a smaller tile), the tile
+// would leave compute units idle: W is dequantised into the workspace instead and the dense plan
+// runs. Packed tile with its own count / with the plan's / this way, us (bf16, rank-16 segment):
+//   512 x 3584 x 3584  53.2 / 132.6 / 32.9     1001 x 3584 x 3584    68.3 / 132.5 / 38.6
+//   512 x 1536 x 8960  57.6 / 90.7 / 35.6      2048 x 1536 x 8960   104.1 / 311.9 / 70.5
+//   257 x 512 x 3584   40.9 / 39.5 / 15.5      4096 x 512 x 3584     57.0 / 132.4 / 27.4
+bool nf4_dense_first(int64_t M, int64_t N, int64_t K) {
+  return M > kNf4Rows && plan_nt(M, N, K).splits != ql_gemm_nf4_auto_splits(M, N, K);
+}
+int64_t nf4_weight_bytes(int64_t N, int64_t K) { return (N * K * 2 + 255) / 256 * 256; }
+int64_t nf4_dense_bytes(int64_t M, int64_t N, int64_t K) {
+  return nf4_weight_bytes(N, K) +
+         ql_gemm_nt_workspace_floats(M, N, plan_nt(M, N, K).splits) * (int64_t)sizeof(float);
+}
+
 }  // namespace
 
 extern "C" int64_t qlora_gemm_nf4_workspace_size(int64_t M, int64_t N, int64_t K) {
   if (M <= kSkinnyMaxRows || N <= 0 || K <= 0 || K % BK) return 0;  // few rows: no split
+  if (nf4_dense_first(M, N, K)) return nf4_dense_bytes(M, N, K);
   return ql_gemm_nt_workspace_floats(M, N, ql_gemm_nf4_auto_splits(M, N, K)) *
          (int64_t)sizeof(float);
 }
@@ -1289,13 +1305,25 @@ extern "C" int qlora_gemm_nf4(int64_t M, int64_t N, int64_t K, const void* A, in
     return ql_gemm_nf4_skinny(M, N, K, A, lda, packed, absmax, nested, code2, absmax2, offset,
                               log2_bs, log2_bs2, nf4_table, K2, A2, lda2, B2, ldb2, in_dtype, C,
                               ldc, bias, alpha, static_cast<hipStream_t>(stream));
+  if (K2 == 0) A2 = B2 = nullptr;
+  if (nf4_dense_first(M, N, K) && workspace && ql_aligned(workspace, 16) &&
+      workspace_bytes >= nf4_dense_bytes(M, N, K)) {
+    const ql_nf4_weight w{packed, N, K, absmax, code2, absmax2, offset, blocksize, blocksize2,
+                          workspace};
+    const int st = qlora_nf4_dequant_group(&w, 1, nested, nf4_table, in_dtype, stream);
+    if (st != QL_OK) return st;
+    return ql_gemm_nt2(in_dtype, in_dtype, M, N, K, A, lda, workspace, K, A2, lda2, B2, ldb2, K2,
+                       C, ldc, bias, alpha, 0.f, plan_nt(M, N, K).splits,
+                       reinterpret_cast<float*>(static_cast<char*>(workspace) +
+                                                nf4_weight_bytes(N, K)),
+                       static_cast<hipStream_t>(stream));
+  }
   int splits = ql_gemm_nf4_auto_splits(M, N, K);
   const int64_t need = ql_gemm_nt_workspace_floats(M, N, splits) * (int64_t)sizeof(float);
   if (need > workspace_bytes || !workspace || !ql_aligned(workspace, 16)) splits = 1;
   const Nf4Operand op{packed, absmax, absmax2, code2, nf4_table, offset, log2_bs, log2_bs2};
   float* ws = static_cast<float*>(workspace);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (K2 == 0) A2 = B2 = nullptr;
   // B's leading dimension is K: the weight's row length, in weights
 #define QL_NF4_LAUNCH(ITC, BQC)                                                                \
   return launch<ITC, ITC, 8, BQC>(A, lda, nullptr, K, A2, lda2, B2, ldb2, K2, C, ldc, bias, M, \

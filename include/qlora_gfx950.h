@@ -482,13 +482,17 @@ int qlora_gemm_nt_cat_residual(int64_t M, int64_t N, int64_t K, const void* A, i
  * absmax2, offset, blocksize, blocksize2, nf4_table) for n_weights = N * K, rounded to
  * in_dtype: the products see exactly those 16-bit values. Above 32 rows C equals
  * qlora_gemm_nt_cat on the dequantised W bit for bit, and W's packed bytes are read once per
- * 256-row tile of A instead of writing and re-reading a dense 16-bit copy; up to 32 rows a kernel
- * without tiles sums the same products in another order of k.
+ * 256-row tile of A instead of writing and re-reading a dense 16-bit copy, but for more than 256
+ * rows of shapes whose dense product runs another split of K than the 256 x 256 tile wants: there
+ * W is dequantised into the workspace first. Up to 32 rows a kernel without tiles sums the same
+ * products in another order of k.
  * K % 64 == 0; blocksize a power of two >= 64 dividing K (blocksize2 a power of two when
- * nested); K2 % 64 == 0 and K2 <= 128 (the rank-16 LoRA segment, zero-padded to 64 columns,
- * as in qlora_gemm_nt_cat); A, packed 16-B aligned, lda >= K a multiple of 8; A2/B2 as in
+ * nested); K2 0 or 64 (the rank-16 LoRA segment, zero-padded to 64 columns, as in
+ * qlora_gemm_nt_cat); A, packed 16-B aligned, lda >= K a multiple of 8; A2/B2 as in
  * qlora_gemm_nt_cat; in_dtype QL_BF16 or QL_F16. Workspace (16-B aligned,
- * qlora_gemm_nf4_workspace_size bytes) enables split-K for outputs with few 256 x 256 tiles.
+ * qlora_gemm_nf4_workspace_size bytes) enables split-K for outputs with few 256 x 256 tiles and
+ * the dequantisation; with less the call runs unsplit, or without the dequantisation, and the
+ * sums may be grouped otherwise than the dense product's.
  * Replaces: solution/nf4.py:101-102 (dequantize_nf4 + F.linear in NF4Linear.forward) together
  * with solution/lora.py:49-60,172 (the adapter GEMMs and the scaled add).
  */

@@ -339,3 +339,14 @@ def test_wgrad_masked_rejects_bad_arguments(lib):
     assert call(bits=null) == -1 and call(slots=5) == -1
     assert call(bits=bad) == -3
     assert call(gs=504) == -4 and call(gs=516) == -4 and call(N=500, gs=512) == -4
+
+
+def test_nf4_gemm_asks_for_the_dequantised_weight_where_the_dense_plan_splits_otherwise(lib):
+    """512 x 3584 x 3584: the dense product runs unsplit on smaller tiles, the packed 256 x 256
+    tile wants 7 splits; up to 256 rows and where the counts agree only partials are asked for."""
+    size = lib.qlora_gemm_nf4_workspace_size
+    assert size(512, 3584, 3584) >= 2 * 3584 * 3584 + lib.qlora_gemm_nt_cat_workspace_size(
+        512, 3584, 3584)
+    assert size(4096, 18944, 3584) == 0
+    assert size(256, 3584, 3584) == lib.qlora_gemm_nt_cat_workspace_size(256, 3584, 3584) > 0
+    assert size(32, 3584, 3584) == 0
