@@ -25,6 +25,7 @@ _c_ptr = ctypes.c_void_p
 _c_f32 = ctypes.c_float
 _c_u64 = ctypes.c_uint64
 _c_i64p = ctypes.POINTER(ctypes.c_int64)
+_c_intp = ctypes.POINTER(ctypes.c_int)
 
 # name -> argtypes; every function returns int (QL_OK = 0)
 _SIGNATURES = {
@@ -96,6 +97,7 @@ _SIGNATURES = {
     "qlora_nf4_dequant_group": [_c_ptr, _c_int, _c_int, _c_ptr, _c_int, _c_ptr],
     "qlora_nf4_dequant_t_group": [_c_ptr, _c_int, _c_int, _c_ptr, _c_i64, _c_int, _c_ptr],
     "qlora_transpose16": [_c_ptr, _c_i64, _c_i64, _c_i64, _c_ptr, _c_i64, _c_ptr],
+    "qlora_gemm_nt_plan": [_c_i64, _c_i64, _c_i64, _c_intp, _c_intp, _c_intp],
     "qlora_gemm_nt_cat": [_c_i64, _c_i64, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_i64, _c_ptr,
                           _c_i64, _c_ptr, _c_i64, _c_int, _c_ptr, _c_i64, _c_int, _c_ptr, _c_f32,
                           _c_ptr, _c_i64, _c_ptr],

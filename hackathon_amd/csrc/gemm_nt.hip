@@ -1098,6 +1098,11 @@ namespace {
 // CU at 0.36; and the two small tiles, which keep fewer loads in flight, lose a quarter where the operands are past what the
 // 256 MB cache holds beside its other work (64 x 128 at 512 x 18944 x 3584: 118 us). A smaller
 // tile is taken only where the model gives it 5%.
+// Long loops (48 steps or more) of the large tile run at 0.88 of its step where they leave a fifth
+// of the CUs idle. That decides against the 128 x 256 tile, split to fill the chip (us, 256-row
+// tile : 128 x 256 in 4 splits): 4096 x 1536 x 8960 124 : 137, 2798 x 2048 x 8960 122 : 130,
+// 757 x 8192 x 8960 129 : 144, 1145 x 8960 x 18944 402 : 429. The 128 x 128 tile gains from idle
+// CUs too (3205 x 1152 x 18944 161 : 139, modelled 189 : 176), so it is compared without.
 struct Plan {
   QlGemmTile tile;
   int splits;
@@ -1107,11 +1112,12 @@ double reduce_us(int64_t M, int64_t N, int s) {
   return s > 1 ? 3.0 + (s + 0.5) * double(M) * double(N) * 4.0 / 6.0e6 : 0.0;
 }
 
-double big_us(int64_t M, int64_t N, int64_t K, int s) {
+double big_us(int64_t M, int64_t N, int64_t K, int s, bool idle = false) {
   const int nb = choose_nb(M, N);
   const int64_t wgs = (M + BM - 1) / BM * ((N + 32 * nb - 1) / (32 * nb)) * s;
   const double steps = double((K / BK + s - 1) / s);
-  return 3.0 + double((wgs + kCUs - 1) / kCUs) * (steps * (nb == 8 ? 1.58 : 1.43) + 6.0) +
+  const double part = idle && steps >= 48 && wgs * 10 <= kCUs * 8 ? 0.88 : 1.0;
+  return 3.0 + double((wgs + kCUs - 1) / kCUs) * (steps * part * (nb == 8 ? 1.58 : 1.43) + 6.0) +
          (s > 1 ? 12.0 : 0.0) + reduce_us(M, N, s);
 }
 
@@ -1144,12 +1150,13 @@ constexpr int64_t kNf4Rows = 256;
 Plan plan_nt(int64_t M, int64_t N, int64_t K) {
   Plan best{QlGemmTile::k256, auto_splits_bn(M, N, K, 32 * choose_nb(M, N))};
   double us = 0.95 * big_us(M, N, K, best.splits);
+  const double us_idle = 0.95 * big_us(M, N, K, best.splits, true);
   const int fixed = best.splits;
   for (const QlGemmTile tile : {QlGemmTile::k128x128, QlGemmTile::k64x128, QlGemmTile::k128x256})
     for (int s = M <= kNf4Rows ? fixed : 1; s <= (M <= kNf4Rows ? fixed : 16); ++s) {
       if (s > 1 && M > kNf4Rows && K / BK / s < 6) break;
       const double t = mid_us(tile, M, N, K, s);
-      if (t < us) {
+      if (t < us && (tile != QlGemmTile::k128x256 || t < us_idle)) {
         us = t;
         best = {tile, s};
       }
@@ -1161,6 +1168,18 @@ Plan plan_nt(int64_t M, int64_t N, int64_t K) {
 
 int ql_gemm_nt_auto_splits(int64_t M, int64_t N, int64_t K, bool accumulate) {
   return accumulate ? auto_splits_bn(M, N, K, 32 * choose_nb(M, N)) : plan_nt(M, N, K).splits;
+}
+
+extern "C" int qlora_gemm_nt_plan(int64_t M, int64_t N, int64_t K, int* tile_m, int* tile_n,
+                                  int* splits) {
+  if (!tile_m || !tile_n || !splits) return QL_EINVAL;
+  if (M <= 0 || N <= 0 || K <= 0 || K % BK) return QL_ESHAPE;
+  const Plan plan = plan_nt(M, N, K);
+  const bool big = plan.tile == QlGemmTile::k256;
+  *tile_m = big ? BM : plan.tile == QlGemmTile::k64x128 ? 64 : 128;
+  *tile_n = big ? 32 * choose_nb(M, N) : plan.tile == QlGemmTile::k128x256 ? 256 : 128;
+  *splits = plan.splits;
+  return QL_OK;
 }
 
 // The packed operand's only tile is 256 x 256, and this its split count.

@@ -141,6 +141,14 @@ def frozen_as(w: torch.Tensor, dtype) -> torch.Tensor:
     return _frozen(w, dtype, lambda t: t.to(dtype).contiguous())
 
 
+def nt_plan(m: int, n: int, k: int) -> tuple[int, int, int]:
+    """(tile rows, tile columns, splits of K) of the NT GEMM for these sizes
+    (qlora_gemm_nt_plan)."""
+    out = [ctypes.c_int() for _ in range(3)]
+    _lib.call("qlora_gemm_nt_plan", m, n, k, *[ctypes.byref(o) for o in out])
+    return tuple(o.value for o in out)
+
+
 def gemm_nt_cat(a: torch.Tensor, b: torch.Tensor, a2: torch.Tensor | None,
                 b2: torch.Tensor | None, out: torch.Tensor, bias: torch.Tensor | None = None,
                 alpha: float = 1.0, residual: torch.Tensor | None = None) -> torch.Tensor:

@@ -440,6 +440,12 @@ int qlora_transpose16(const void* in, int64_t rows, int64_t cols, int64_t ld_in,
                       int64_t ld_out, ql_stream_t stream);
 
 /*
+ * The output tile and the split of K that qlora_gemm_nt_cat (and qlora_gemm_ws with beta 0) runs
+ * for these sizes when its workspace suffices; host only. K % 64 == 0 (else QL_ESHAPE).
+ */
+int qlora_gemm_nt_plan(int64_t M, int64_t N, int64_t K, int* tile_m, int* tile_n, int* splits);
+
+/*
  * NT GEMM over two concatenated K segments (bf16/fp16 operands, fp32 accumulation):
  *   C[M,N] = alpha * (A[M,K] B[N,K]^T + A2[M,K2] B2[N,K2]^T) (+ bias[n])
  * K and K2 multiples of 64, one of them at most 128 (QL_ESHAPE otherwise); all four operands
