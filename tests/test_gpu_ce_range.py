@@ -65,3 +65,29 @@ def test_a_nan_reaches_the_loss_and_its_row_only():
     assert torch.equal(pred[[0, 1, 3]], z[[0, 1, 3]].argmax(1))
     ref = ops.ce_rows(z[:2], t[:2], 1, grad_scale=3.0)
     torch.testing.assert_close(loss[:2].double(), ref[0], rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("V", [1, 7, 511, 513, 2047, 2049, 2561, 4097])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_element_rows_around_whole_pieces(V, dtype):
+    """Rows that go element by element, on both sides of one element and of one piece of four for
+    each of the 512 threads."""
+    print(f"ce element rows V={V} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(V)
+    z = torch.randn(5, V, generator=g).to(dtype)
+    t = torch.randint(0, V, (5,), generator=g)
+    t[2] = -100
+    lse = torch.logsumexp(z.double(), 1)
+    lab = t >= 0
+    at = z.double().gather(1, t.clamp(min=0)[:, None])[:, 0]
+    zg = z.cuda()
+    loss, ent, cor, pred = _rows(zg, t.cuda())
+    torch.testing.assert_close(loss.double(), torch.where(lab, lse - at, 0.0), rtol=1e-4, atol=1e-4)
+    p = torch.softmax(z.double(), 1)
+    logp = torch.log_softmax(z.double(), 1)
+    torch.testing.assert_close(ent.double(), -(p * logp).sum(1), rtol=1e-4, atol=1e-4)
+    assert torch.equal(pred, (z.double() == z.double().max(1, keepdim=True).values).int().argmax(1))
+    p[torch.arange(5), t.clamp(min=0)] -= lab.double()
+    dz = p * 3.0 * lab.double()[:, None]
+    tol = 1e-2 if dtype == torch.bfloat16 else 4e-5
+    torch.testing.assert_close(zg.cpu().double(), dz.to(dtype).double(), rtol=tol, atol=tol)
