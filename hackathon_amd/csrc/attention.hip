@@ -951,12 +951,24 @@ void attn_bwd_dq(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
 
 // Query tiles of 16 rows per wave in the forward and dQ kernels (64 QT query rows per
 // workgroup). 128 rows read K and V from LDS half as often per product; 64 rows make twice the
-// workgroups, each with about 0.6 of the latency per key block, and win while 128 rows leave a
-// compute unit fewer than its two workgroups. Forward / backward in us, 128 against 64 rows:
+// workgroups, each with about 0.6 of the latency per key block. So 64 rows win while their
+// workgroups all run at once, two per compute unit, and beyond that while 128 rows leave a compute
+// unit fewer than its two workgroups and the causal items of a head differ enough in work for the
+// smaller ones to even out. Forward / backward in us, 128 against 64 rows:
 //   84 items of 128 rows 13.1 / 39.2 : 9.9 / 34.7     216: 23.5 / 63.1 : 18.5 / 57.6
 //   256: 28.0 / 69.4 : 21.6 / 62.6   384 (S = 4096): 89.0 / 235 : 71.2 / 224
-//   448: 49.9 / 150 : 45.1 / 147     512: 50.5 / 160 : 49.9 / 163    576: 53.6 / 180 : 57.9 / 188
-int query_tiles(int64_t bh, int64_t S) { return bh * ((S + 127) / 128) < 2 * kUnits ? 1 : 2; }
+//   448 (S = 2048): 49.9 / 150 : 45.1 / 147     512: 50.5 / 160 : 49.9 / 163
+//   576: 53.6 / 180 : 57.9 / 188
+// and with few blocks a head, time with 64 rows over time with 128 (heads x S): 168 x 192 0.77,
+// 0.90; 168 x 256 0.99, 0.98; 84 x 512 0.91, 0.97; 56 x 777 0.87, 0.95; 56 x 1024 0.95, 1.00; but
+// 280 x 65 1.27, 1.05; 448 x 100 1.14, 1.05; 500 x 128 1.24, 1.08; 224 x 129 1.20, 1.04;
+// 112 x 512 1.05, 1.02; 168 x 384 1.17, 1.05.
+int query_tiles(int64_t bh, int64_t S) {
+  const int64_t blocks = (S + 127) / 128, items = bh * blocks;  // of 128 rows
+  if (bh * ((S + 63) / 64) <= 2 * kUnits) return 1;
+  if (blocks >= 2 && items <= 3 * kUnits / 2) return 1;
+  return blocks >= 7 && items < 2 * kUnits ? 1 : 2;
+}
 
 int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
 

@@ -58,3 +58,10 @@ def test_row_strides_around_the_whole_tile_loads(row_stride):
     got += tuple(attention.attn_bwd(*far, *got, do, scale))
     for name, a, b in zip(("o", "lse", "dq", "dk", "dv"), got, want):
         assert torch.equal(a, b), name
+
+
+# (heads, length): more than two 64-row workgroups per compute unit with few blocks a head, where
+# 128 rows are taken from fewer items than two per unit
+@pytest.mark.parametrize("H,S", [(280, 65), (448, 100), (224, 129), (112, 512), (168, 383)])
+def test_many_short_heads(H, S):
+    test_every_item_is_taken_once(H, S, torch.bfloat16)
