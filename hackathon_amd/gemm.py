@@ -61,7 +61,10 @@ def gemm(a: torch.Tensor, b: torch.Tensor, *, a_km: bool = False, b_kn: bool = F
         # B stored [K, N]: one tiled transpose (2·K·N·2 bytes of traffic) puts it k-contiguous,
         # and the large-tile NT kernel then runs at about twice the general kernel's rate
         b, b_kn = transpose16(b), False
-    ws_bytes = int(_lib.load().qlora_gemm_workspace_size(int(a_km), int(b_kn), M, N, K))
+    if beta == 0 and not a_km and not b_kn:  # the plain plan's partials alone
+        ws_bytes = int(_lib.load().qlora_gemm_nt_cat_workspace_size(M, N, K))
+    else:
+        ws_bytes = int(_lib.load().qlora_gemm_workspace_size(int(a_km), int(b_kn), M, N, K))
     ws = torch.empty((ws_bytes + 3) // 4, dtype=torch.float32, device=out.device) \
         if ws_bytes > 0 else None
     _lib.call("qlora_gemm_ws", int(a_km), int(b_kn), M, N, K, a.data_ptr(), a.stride(0),

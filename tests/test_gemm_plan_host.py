@@ -1,8 +1,9 @@
 """Which tile and split of K the NT GEMM takes (qlora_gemm_nt_plan), on the host."""
 
 import pytest
+import torch
 
-from hackathon_amd import gemm
+from hackathon_amd import _lib, gemm
 
 
 @pytest.mark.parametrize("M,N,K", [(4096, 1536, 8960), (757, 8192, 8960), (2798, 2048, 8960),
@@ -26,3 +27,19 @@ def test_sizes_the_kernel_does_not_take_are_refused():
     for sizes in ((0, 64, 64), (64, 0, 64), (64, 64, 0), (64, 64, 96)):
         with pytest.raises(RuntimeError, match="inconsistent sizes"):
             gemm.nt_plan(*sizes)
+
+
+@pytest.mark.parametrize("M,N,K", [(4096, 512, 3584), (1001, 3584, 3584), (512, 512, 4096)])
+def test_plain_products_ask_for_their_own_partials_only(monkeypatch, M, N, K):
+    """The accumulating plan's splits (7 of 4096 x 512: 59 MB) are not allocated where beta is 0."""
+    plan = gemm.nt_plan(M, N, K)[2]
+    asked = []
+    monkeypatch.setattr(_lib, "call", lambda name, *a: asked.append(a[-2]))
+    monkeypatch.setattr(_lib, "require_device", lambda *t: None)
+    monkeypatch.setattr(_lib, "stream_of", lambda t: 0)
+    a, b = torch.empty(M, K, dtype=torch.bfloat16), torch.empty(N, K, dtype=torch.bfloat16)
+    out = torch.empty(M, N, dtype=torch.bfloat16)
+    gemm.gemm(a, b, out=out)
+    gemm.gemm(a, b, out=out, beta=1.0)
+    assert asked[0] == (plan * M * N * 4 if plan > 1 else 0)
+    assert asked[1] == _lib.load().qlora_gemm_workspace_size(0, 0, M, N, K) > 0
