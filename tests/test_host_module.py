@@ -34,6 +34,11 @@ def test_cpu_and_mistyped_operands_raise():
         host.group_forward(x, a16, bs, weights, None, 0.0, [], None, 0)
 
 
+def test_stream_of_a_tensor_off_the_gpu_raises():
+    with pytest.raises(ValueError, match="on a GPU device"):
+        _lib.stream_of(torch.zeros(1))
+
+
 def test_weight_args_hold_a_contiguous_copy_of_strided_codes():
     w = torch.randn(64, 128)
     packed, qs = quant.quantize_nf4(w, 64)
