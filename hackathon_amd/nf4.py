@@ -18,7 +18,7 @@ from __future__ import annotations
 
 import torch
 
-from . import _lib
+from . import _host, _lib
 from . import gemm as _gemm
 from . import quant
 
@@ -269,36 +269,19 @@ LORA_FEW_MAX_ROWS = 32  # qlora_nf4_lora_few's row limit
 def lora_few(x, packed, quant_state, lora_a, lora_b, scaling, bias=None):
     """x @ W^T + bf16(x @ A^T) @ (scaling B)^T (+ bias) for x [M <= 32, K] and an adapter's fp32
     factors A [16, K], B [N, 16], in two launches (qlora_nf4_lora_few)."""
-    M, K = x.shape
-    N, K_w = (int(d) for d in quant_state.shape)
-    if K != K_w:
-        raise ValueError(f"x has {K} columns, the weight {K_w}")
-    if lora_a.shape != (16, K) or lora_b.shape != (N, 16):
-        raise ValueError(f"the factors must be [16, {K}] and [{N}, 16], got "
-                         f"{tuple(lora_a.shape)} and {tuple(lora_b.shape)}")
-    if x.dtype not in (torch.bfloat16, torch.float16) or lora_a.dtype != torch.float32 \
-            or lora_b.dtype != torch.float32:
-        raise TypeError(f"x must be bf16 or fp16 and the factors fp32, got {x.dtype}, "
-                        f"{lora_a.dtype}, {lora_b.dtype}")
-    if x.stride(-1) != 1 or not (lora_a.is_contiguous() and lora_b.is_contiguous()
-                                 and packed.is_contiguous()):
-        raise ValueError("x must have unit stride along its rows; the factors and the packed "
-                         "codes must be contiguous")
-    if packed.numel() * packed.element_size() * 2 < N * K:
-        raise ValueError("packed buffer is smaller than the quantised shape")
+    M = x.shape[0]
+    N, K = quant_state.shape
     if bias is not None:
-        if bias.numel() != N:
-            raise ValueError(f"bias has {bias.numel()} elements, the output {N} columns")
         bias = bias.to(x.dtype).contiguous()
-    _lib.require_device(x, packed, lora_a, lora_b, bias)
+    x_p, packed_p, a_p, b_p, bias_p = _host.load().few_rows_operands(x, packed, lora_a, lora_b,
+                                                                     bias, N, K)
     absmax, nested, code2, absmax2, offset, blocksize2 = _scale_args(quant_state)
     out = torch.empty((M, N), dtype=x.dtype, device=x.device)
     ws, ws_bytes = _lib.workspace("qlora_nf4_lora_few_workspace_size", M, K, device=x.device)
-    _lib.call("qlora_nf4_lora_few", M, N, K, x.data_ptr(), x.stride(0), packed.data_ptr(),
-              absmax.data_ptr(), nested, _lib.ptr(code2), _lib.ptr(absmax2), offset,
-              int(quant_state.blocksize), blocksize2, _nf4_table(packed.device).data_ptr(),
-              lora_a.data_ptr(), lora_b.data_ptr(), float(scaling), _lib.tag(x.dtype),
-              out.data_ptr(), N, _lib.ptr(bias), _lib.ptr(ws), ws_bytes, _lib.stream_of(x))
+    _lib.call("qlora_nf4_lora_few", M, N, K, x_p, x.stride(0), packed_p, absmax.data_ptr(), nested,
+              _lib.ptr(code2), _lib.ptr(absmax2), offset, int(quant_state.blocksize), blocksize2,
+              _nf4_table(x.device).data_ptr(), a_p, b_p, float(scaling), _lib.tag(x.dtype),
+              out.data_ptr(), N, bias_p, _lib.ptr(ws), ws_bytes, _lib.stream_of(x))
     return out
 
 

@@ -2,8 +2,6 @@
 rows) refuse operands their kernels would read out of range, before any launch; the launches are
 recorded instead of made."""
 
-import ctypes
-
 import pytest
 import torch
 
@@ -17,7 +15,6 @@ def launches(monkeypatch):
     calls = []
     monkeypatch.setattr(_lib, "call", lambda *a: calls.append(a))
     monkeypatch.setattr(_lib, "stream_of", lambda t: 0)
-    monkeypatch.setattr(_lib, "require_device", lambda *t: None)
     return calls
 
 
@@ -27,10 +24,23 @@ def _operands():
     return x, packed, qs, torch.randn(16, K), torch.randn(N, 16)
 
 
-def test_operands_that_fit_are_launched(launches):
-    x, packed, qs, a, b = _operands()
-    assert nf4.lora_few(x, packed, qs, a, b, 2.0).shape == (2, N)
-    assert [c[0] for c in launches] == ["qlora_nf4_lora_few"]
+def test_operands_that_fit_are_launched(launches, monkeypatch):
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    _, _, qs, _, _ = _operands()
+    monkeypatch.setattr(nf4, "_nf4_table", lambda device: torch.zeros(16))
+    with FakeTensorMode():  # a GPU's device, no storage
+        t = lambda *shape, dtype: torch.empty(*shape, dtype=dtype, device="cuda:0")  # noqa: E731
+        monkeypatch.setattr(nf4, "_scale_args", lambda qs: (t(128, dtype=torch.uint8), 0, None,
+                                                            None, 0.0, 1))
+        monkeypatch.setattr(_lib, "workspace", lambda *a, device: (None, 0))
+        monkeypatch.setattr(torch.Tensor, "data_ptr", lambda self: 0)
+        for bias in (None, t(N, dtype=torch.bfloat16), t(N, dtype=torch.float32)):
+            y = nf4.lora_few(t(2, K, dtype=torch.bfloat16), t(N * K // 2, dtype=torch.uint8), qs,
+                             t(16, K, dtype=torch.float32), t(N, 16, dtype=torch.float32), 2.0,
+                             bias)
+            assert y.shape == (2, N)
+    assert [c[0] for c in launches] == ["qlora_nf4_lora_few"] * 3
 
 
 @pytest.mark.parametrize("what,error", [
@@ -103,20 +113,32 @@ def test_layer_of_another_width_raises_with_gradients(launches, monkeypatch, p):
     assert not launches
 
 
-def _dense_at(address, n):
-    return torch.frombuffer((ctypes.c_char * (2 * n)).from_address(address),
-                            dtype=torch.bfloat16).clone()
-
-
 def test_strided_bias_reaches_the_few_row_launch_dense(launches, monkeypatch):
     x, packed, qs, a, b = _operands()
     bias = torch.randn(N, 2).bfloat16()[:, 0]
     seen = []
-    monkeypatch.setattr(_lib, "call", lambda *args: seen.append(_dense_at(args[-4], N)))
+
+    class Host:
+        @staticmethod
+        def few_rows_operands(x, packed, a, b, bias, n, k):
+            seen.append(bias)
+            return 0, 0, 0, 0, 0
+
+    monkeypatch.setattr(nf4._host, "load", lambda: Host)
     lora.LoraNF4Few.apply(x, a, b, packed, qs, bias, 2.0)
-    assert torch.equal(seen[0], bias)
-    with pytest.raises(ValueError, match="bias"):
-        lora.LoraNF4Few.apply(x, a, b, packed, qs, bias[:32], 2.0)
+    assert seen[0].is_contiguous() and torch.equal(seen[0], bias)
+
+
+def test_bias_of_another_length_raises():
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    host = lora._host.load()
+    with FakeTensorMode():
+        t = lambda *shape, dtype=torch.float32: torch.empty(*shape, dtype=dtype,  # noqa: E731
+                                                            device="cuda:0")
+        with pytest.raises(ValueError, match="bias must be 64"):
+            host.few_rows_operands(t(2, K, dtype=torch.bfloat16), t(N * K // 2, dtype=torch.uint8),
+                                   t(16, K), t(N, 16), t(32, dtype=torch.bfloat16), N, K)
 
 
 def test_strided_bias_reaches_the_native_calls_dense(launches, monkeypatch):
