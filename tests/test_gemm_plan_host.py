@@ -43,3 +43,20 @@ def test_plain_products_ask_for_their_own_partials_only(monkeypatch, M, N, K):
     gemm.gemm(a, b, out=out, beta=1.0)
     assert asked[0] == (plan * M * N * 4 if plan > 1 else 0)
     assert asked[1] == _lib.load().qlora_gemm_workspace_size(0, 0, M, N, K) > 0
+
+
+def test_the_tile_tests_run_the_tiles_they_name():
+    """The planner's choice for the cases of test_gpu_gemm_mid: refitting it must not leave a tile
+    untested."""
+    from test_gpu_gemm_mid import CASES
+
+    assert [gemm.nt_plan(*c[:3]) for c in CASES] == [
+        (128, 128, 1), (128, 128, 1), (64, 128, 1), (64, 128, 1), (64, 128, 5), (64, 128, 1),
+        (128, 256, 1), (128, 256, 6), (64, 128, 1), (64, 128, 1), (64, 128, 7)]
+
+
+def test_the_large_tile_tests_run_the_large_tile():
+    from test_gpu_gemm_large_tile import CASES
+
+    assert all(gemm.nt_plan(*c[:3]) == c[6] for c in CASES)
+    assert {c[6][1] for c in CASES} == {224, 256} and {c[6][2] for c in CASES} == {1, 3}

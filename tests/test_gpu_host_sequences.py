@@ -4,7 +4,7 @@ operand forms a caller may hand in, against an fp64 product."""
 import pytest
 import torch
 
-from hackathon_amd import lora, nf4, quant
+from hackathon_amd import _host, _lib, gemm, lora, nf4, quant
 
 pytestmark = pytest.mark.gpu
 
@@ -70,3 +70,59 @@ def test_wide_codes_refused_by_the_dense_forward():
     with pytest.raises(ValueError, match="packed buffer is smaller"):
         lora.LoraNF4Linear.apply(x, a, b, packed.view(-1).view(torch.bfloat16), st, None, 2.0,
                                  0.0, 0)
+
+
+def _offset_codes(packed, nbytes):
+    buf = torch.empty(packed.numel() + nbytes, dtype=torch.uint8, device="cuda")
+    buf[nbytes:] = packed.reshape(-1)
+    return buf[nbytes:]
+
+
+@pytest.mark.parametrize("kind", ["alike", "nested and plain", "codes off 4 bytes",
+                                  "codes off 16 bytes"])
+def test_group_and_single_dequantisation_give_the_same_product(kind):
+    """The native group calls dequantise up to four weights that fit the group kernels in one
+    launch, and others one by one: with the adapters zero, the products of the dequantised weights
+    bit for bit."""
+    print(f"native dequantisation: {kind}", flush=True)
+    M, K, N = 300, 256, 192
+    G = 2
+    g = torch.Generator(device="cuda").manual_seed(7)
+    items = []
+    for i in range(G):
+        w = torch.randn(N, K, device="cuda", generator=g) * 0.02
+        packed, st = quant.quantize_nf4(w, 64, compress_statistics=kind != "nested and plain" or i)
+        if kind.startswith("codes off"):
+            packed = _offset_codes(packed, 2 if "4" in kind else 4)
+        items.append((packed, st))
+    x = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    dy = torch.randn(M, G * N, device="cuda", generator=g).bfloat16()
+    z = lambda *s: torch.zeros(*s, device="cuda", dtype=torch.bfloat16)  # noqa: E731
+    host, table, stream = _host.load(), nf4._nf4_table(x.device), _lib.stream_of(x)
+    weights = [nf4.weight_args(*it) for it in items]
+    w = torch.cat([nf4.dequantize_nf4(p, st, torch.bfloat16) for p, st in items])
+    y, _, _ = host.group_forward(x, z(16 * G, K), z(G * N, 64), weights, None, 0.0, [], table,
+                                 stream)
+    want = gemm.gemm_nt_cat(x, w, z(M, 64), z(G * N, 64), z(M, G * N))
+    assert torch.equal(y, want)
+    if kind.startswith("codes off"):
+        return  # the transposed kernel takes codes aligned to 16 bytes only
+    ut = z(16 * G, 304)[:, :M]
+    dx, grads = host.group_backward(dy, x, z(K, 64), z(16 * G, G * N), ut, weights, [1.0] * G, True,
+                                    [False] * (2 * G), None, None, [], 0.0, None, [], table, stream)
+    want = gemm.gemm_nt_cat(dy, w.t().contiguous(), z(M, 64), z(K, 64), z(M, K))
+    assert torch.equal(dx, want) and grads == [None] * (2 * G)
+
+
+def test_codes_off_16_bytes_are_refused_by_the_transposed_dequantisation():
+    g, packed, st, a, b = _layer(256, 128, 2)
+    x = torch.randn(300, 128, device="cuda", generator=g).bfloat16()
+    t = torch.zeros(16, 256, device="cuda", dtype=torch.bfloat16)
+    at = torch.zeros(128, 64, device="cuda", dtype=torch.bfloat16)
+    dy = torch.randn(300, 256, device="cuda", generator=g).bfloat16()
+    with pytest.raises(RuntimeError, match="alignment"):
+        _host.load().group_backward(dy, x, at, t, torch.zeros(16, 304, device="cuda",
+                                                              dtype=torch.bfloat16)[:, :300],
+                                    [nf4.weight_args(_offset_codes(packed, 4), st)], [1.0], True,
+                                    [False, False], None, None, [], 0.0, None, [],
+                                    nf4._nf4_table(x.device), _lib.stream_of(x))
