@@ -1143,8 +1143,9 @@ double mid_us(QlGemmTile tile, int64_t M, int64_t N, int64_t K, int s) {
 }
 
 // Up to this many rows the split count is the 256-row tile's, whatever tile runs: there the
-// forward multiplies by the packed NF4 weight (qlora_gemm_nf4, 256 x 256 tiles), and the same
-// product of the dequantised weight has to be the same sum.
+// forward multiplies by the packed NF4 weight (qlora_gemm_nf4, from 33 rows on with 256 x 256
+// tiles), and the same product of the dequantised weight has to be the same sum. (Up to 32 rows the
+// packed product has a kernel that sums k in another order, so there nothing hangs on the count.)
 constexpr int64_t kNf4Rows = 256;
 
 Plan plan_nt(int64_t M, int64_t N, int64_t K) {

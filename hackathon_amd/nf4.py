@@ -169,7 +169,8 @@ def _group_call(name, items, outs, dtype, *extra):
 
 def dequantize_nf4_group(items, dtype, outs):
     """Dequantise the weights `items` = [(packed, quant_state), ...] into `outs` (one
-    contiguous [out_features, in_features] tensor of `dtype` each): one launch for up to four
+    contiguous [out_features, in_features] tensor of `dtype` each; the fused layers queue the same
+    entry from native code): one launch for up to four
     weights of the same nesting (qlora_nf4_dequant_group), else one dequantize_nf4 each.
     Bit-identical either way."""
     for out in outs:
@@ -197,9 +198,11 @@ def dequantize_nf4_t_group(items, dtype, outs):
 
 
 # Token rows up to which the forward GEMM dequantises W inside the GEMM (gemm_nf4) instead of
-# writing a dense 16-bit W first. Measured on MI355X at the Qwen2.5-7B projection shapes: the
-# fused GEMM is 1.12-1.28x faster at 64 and 256 rows (W's dense write and re-read dominate),
-# 0.83-0.98x at 512 and 0.63-0.72x at 4096 (every 256-row tile of x redoes the dequantisation).
+# writing a dense 16-bit W first. Measured on MI355X, gemm_nf4 against dequantisation and dense
+# GEMM, us at 64 / 256 rows: 18944 x 3584 60 : 63 / 81 : 103, 3584 x 18944 58 : 64 / 84 : 110 (W's
+# dense write and re-read dominate). Narrower weights, whose dense product takes tiles smaller than
+# the packed one's 256 x 256, are faster dequantised first at every count above 32: 3584 x 3584
+# 33 : 24 / 50 : 32, 4864 x 896 38 : 15 / 39 : 16. One limit for all shapes does not follow that.
 FUSED_GEMM_MAX_ROWS = 256
 
 
@@ -239,9 +242,10 @@ def fused_gemm_ok(quant_state, packed, x=None, a2=None):
 
 def gemm_nf4(x, packed, quant_state, out=None, a2=None, b2=None, bias=None, alpha=1.0):
     """out = alpha * (x @ W^T + a2 @ b2^T) (+ bias) with W [N, K] the NF4 weight of
-    `quant_state`, dequantised inside the GEMM to x's dtype (bit-identical to the GEMM on
-    dequantize_nf4(packed, quant_state, x.dtype)); a2 [M, K2] and b2 [N, K2] are the optional
-    rank-16 segment (K2 = 64: one K step) (qlora_gemm_nf4). x [M, K] 2-D."""
+    `quant_state`, dequantised inside the GEMM to x's dtype; a2 [M, K2] and b2 [N, K2] are the
+    optional rank-16 segment (K2 = 64: one K step) (qlora_gemm_nf4). x [M, K] 2-D. From 33 rows on
+    bit-identical to the GEMM on dequantize_nf4(packed, quant_state, x.dtype); up to 32 rows the
+    same products summed in another order of k (the last bit may differ)."""
     _lib.require_device(x, packed)
     N, K = tuple(quant_state.shape)
     M = x.shape[0]
@@ -268,7 +272,9 @@ LORA_FEW_MAX_ROWS = 32  # qlora_nf4_lora_few's row limit
 
 def lora_few(x, packed, quant_state, lora_a, lora_b, scaling, bias=None):
     """x @ W^T + bf16(x @ A^T) @ (scaling B)^T (+ bias) for x [M <= 32, K] and an adapter's fp32
-    factors A [16, K], B [N, 16], in two launches (qlora_nf4_lora_few)."""
+    factors A [16, K], B [N, 16], in two launches (qlora_nf4_lora_few). The down-projection's sums
+    are grouped otherwise than LoraNF4Linear's, so a layer's output for few rows may differ in the
+    last bit between calls with and without gradients."""
     M = x.shape[0]
     N, K = quant_state.shape
     if bias is not None:

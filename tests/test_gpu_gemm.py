@@ -84,10 +84,11 @@ def test_gemm_output_view_with_row_stride():
                                    (4000, 4608, 128)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_gemm_nt_large_tile_edges(M, N, K, dtype):
-    """k-contiguous operands with K % 64 == 0 take the large-tile kernel (256 x 256, or
-    256 x 224 when N is a multiple of 224 and it fills the CUs better: the 4096 and 4000 x 3584
-    cases take 224, the 4000-row ones with a ragged last row of tiles); M and N edges are
-    loaded clamped and must never be stored."""
+    """k-contiguous operands with K % 64 == 0 take a tiled kernel: the 4096- and 4000-row cases the
+    large tile (256 x 256, or 256 x 224 when N is a multiple of 224 and it fills the CUs better:
+    the x 3584 cases; the 4000-row ones with a ragged last row of tiles), the others the smaller
+    tiles (test_gpu_gemm_large_tile has the large tile's ragged sizes); M and N edges are loaded
+    clamped and must never be stored."""
     print(f"gemm_nt M={M} N={N} K={K} {dtype}", flush=True)
     g = torch.Generator().manual_seed(M + 11 * N + K)
     a = torch.randn(M, K, generator=g).to(dtype)
@@ -120,7 +121,9 @@ def test_gemm_nt_bias_alpha_beta_large_tile(N):
                                    (100, 70, 4096), (256, 3584, 8192)])
 def test_gemm_split_k_matches_and_is_deterministic(M, N, K):
     """Small outputs with long K are split over K into an fp32 workspace and summed in split
-    order: the result is within the fp32-accumulation bound and identical run to run."""
+    order (on the smaller tiles; 4096 x 512 x 3584 runs unsplit there): the result is within the
+    fp32-accumulation bound and identical run to run. The size query covers accumulating calls,
+    which split in every case."""
     from hackathon_amd import _lib
 
     print(f"gemm split-K M={M} N={N} K={K}", flush=True)
@@ -163,7 +166,7 @@ def test_transposed_frozen_cache_follows_the_weight():
                                       (4096, 4608, 256, 64), (300, 256, 64, 320),
                                       (256, 3584, 128, 1024)])
 def test_gemm_nt_cat(M, N, K, K2):
-    """a b^T + a2 b2^T over the concatenated K in one GEMM (split-K included for 4096x512; a
+    """a b^T + a2 b2^T over the concatenated K in one GEMM (a
     second segment longer than 128 with a first of at most 128 swaps their roles)."""
     print(f"gemm_nt_cat M={M} N={N} K={K} K2={K2}", flush=True)
     g = torch.Generator().manual_seed(M + N + K + K2)

@@ -1,9 +1,9 @@
 """The decoder layer's last add taken into the down projection's GEMM
 (qlora_gemm_nt_cat_residual, fused_proj.LoraMLP with a residual).
 
-Bar: bit-identical to the GEMM followed by torch's `residual + out` on every epilogue the GEMM
-has (the LDS-staged tile store, the direct store for a row length that is not a multiple of
-8, the split-K reduce), and a model's loss and adapter gradients bit-identical with and
+Bar: bit-identical to the GEMM followed by torch's `residual + out` on the large tile (the
+4096-row case; test_gpu_gemm_large_tile has its ragged, direct-store and split-K forms) and on the
+smaller tiles (the others), and a model's loss and adapter gradients bit-identical with and
 without the fusion.
 """
 
