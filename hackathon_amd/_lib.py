@@ -233,9 +233,12 @@ def stream_of(t: torch.Tensor) -> int:
     """The handle of the current stream of t's device (torch.cuda.current_stream builds a Stream
     object around it, 1.9 us against 0.1 a launch). A tensor off the GPU raises ValueError, as it
     did there."""
-    if not t.is_cuda:
-        raise ValueError(f"expected a tensor on a GPU device, got one on {t.device}")
-    return torch._C._cuda_getCurrentRawStream(t.device.index)
+    try:
+        return torch._C._cuda_getCurrentRawStream(t.device.index)
+    except RuntimeError:
+        if t.is_cuda:
+            raise
+        raise ValueError(f"expected a tensor on a GPU device, got one on {t.device}") from None
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
