@@ -214,6 +214,10 @@ def lora_t_buffer(m: int, dtype, device, rows: int = 16) -> torch.Tensor:
     return torch.empty((rows, (m + 7) // 8 * 8), dtype=dtype, device=device)[:, :m]
 
 
+# The adapter gradients as calls of their own: the fused layers queue the same entries from native
+# code (csrc/host/host.cpp).
+
+
 def lora_wgrad_diag(pt: torch.Tensor, q: torch.Tensor, col_offsets, alphas) -> torch.Tensor:
     """The lora_B gradients of G adapters with concatenated outputs from one pass: fp32 [N, 16]
     whose rows off_i .. off_{i+1} - 1 are alphas[i] * q[:, off_i:off_{i+1}]^T pt[16 i:16 i + 16]^T

@@ -158,6 +158,10 @@ def keep_bits_buffer(M, K, device):
     return torch.empty(((M + 7) // 8, K), dtype=torch.uint8, device=device)
 
 
+# dropout_with_bits, up_masked_add and up_masked_add_slots are calls of their own: the fused layers
+# queue the dropout entries from native code (csrc/host/host.cpp).
+
+
 def dropout_with_bits(x2, p, seed):
     """(x2 * keep / (1 - p), keep bits in keep_bits_buffer's layout) in x2's dtype, the mask of
     DropoutCast(x2, p, seed) (qlora_lora_dropout_scale_bits)."""
